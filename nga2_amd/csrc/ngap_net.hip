@@ -23,188 +23,406 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
 __device__ __forceinline__ int wrapi(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
 
-// output tile of one workgroup: 16 x 4 x 4 voxels, 4 waves (one z-slice each)
+// Linear workgroup id remapped so that each of the 8 XCDs (workgroup b runs on
+// XCD b % 8) walks one contiguous range: neighbouring tiles share the halo
+// voxels in one L2. Bijective on [0, nb).
+__device__ __forceinline__ int xcd_order(int b, int nb) {
+    const int q = nb >> 3, r = nb & 7;
+    const int x = b & 7, m = b >> 3;
+    return x < r ? x * (q + 1) + m : r * (q + 1) + (x - r) * q + m;
+}
+
+// output tile of one workgroup: 16 x TY x 4 voxels, 4 waves (one z-slice each)
 constexpr int TXV = 16, TYV = 4, TZV = 4;
-constexpr int HX = TXV + 2, HY = TYV + 2, HZ = TZV + 2;
-constexpr int HVOX = HX * HY * HZ;  // 648 halo voxels
-constexpr int CK = 32;              // channel chunk
-constexpr int IN_STRIDE = 40;       // bf16 per halo voxel row in LDS (80 B: 16-B aligned, fewer bank conflicts)
-constexpr int W_STRIDE = 40;        // bf16 per weight row (co) in LDS
+constexpr int CK = 32;  // channel chunk
+
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------- forward 3x3x3
-// grid.x = tiles, grid.y = Cout/32. Writes FP32 pre-activations (out32, may be
-// null) and/or BF16 ReLU(out) (outb, may be null).
-__global__ void __launch_bounds__(256) k_conv3_fwd(const __bf16 *__restrict__ in, const __bf16 *__restrict__ wt,
-                                                   float *__restrict__ out32, __bf16 *__restrict__ outb, int nx,
-                                                   int ny, int nz, int cin, int cout, int relu) {
-    // weights are staged one plane of taps (9 of 27) at a time, so the tile
-    // takes 41 + 18 KB of LDS and two workgroups fit on a CU
-    __shared__ __attribute__((aligned(16))) __bf16 s_in[HVOX * IN_STRIDE];
-    __shared__ __attribute__((aligned(16))) __bf16 s_w[9 * CK * W_STRIDE];
-    const int tilesx = nx / TXV, tilesy = ny / TYV;
-    const int t = blockIdx.x;
-    const int x0 = (t % tilesx) * TXV;
-    const int y0 = ((t / tilesx) % tilesy) * TYV;
-    const int z0 = (t / (tilesx * tilesy)) * TZV;
-    const int co0 = blockIdx.y * CK;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    f32x4 acc[TYV][2];
-    for (int a = 0; a < TYV; a++)
-        for (int b = 0; b < 2; b++) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int lrow = lane & 15, lk = (lane >> 4) * 8;
-    for (int ci0 = 0; ci0 < cin; ci0 += CK) {
-        // stage the halo tile: 648 voxels x 32 channels, 16 B per piece
-        for (int q = tid; q < HVOX * 4; q += 256) {
-            const int hv = q >> 2, part = q & 3;
-            const int hx = hv % HX, hy = (hv / HX) % HY, hz = hv / (HX * HY);
-            const int gx = wrapi(x0 - 1 + hx, nx), gy = wrapi(y0 - 1 + hy, ny), gz = wrapi(z0 - 1 + hz, nz);
-            const long long gv = (long long)gx + (long long)nx * (gy + (long long)ny * gz);
-            const uint4 val = *reinterpret_cast<const uint4 *>(in + gv * cin + ci0 + part * 8);
-            *reinterpret_cast<uint4 *>(s_in + hv * IN_STRIDE + part * 8) = val;
+// Implicit GEMM: M = 16 output channels (two blocks per workgroup), N = 16
+// voxels along x, K = 32 input channels of one tap. A workgroup stages the halo
+// tile of a 32-channel chunk in LDS, 64 bytes per voxel with the four 16-byte
+// pieces rotated by (x / 2) % 4, so that the 16-byte reads of consecutive
+// voxels fall on different banks without padding.
+//
+// With one LDS read per tap and operand the kernel was bound by the LDS read
+// rate and by the staging between barriers. So a halo row is read once per
+// (dz, dx) and used for the three taps dy of three output rows (TY + 2 reads
+// for 6 TY MFMAs); the weights do not pass through LDS: each wave loads its six
+// operands of the next (dz, dx) from L1/L2 while it works on this one; and a
+// workgroup walks over several tiles, with the next tile's (or chunk's) halo
+// on its way to registers behind the products. TY = 8 takes 69 KB of LDS: two
+// workgroups per CU. The sched_barriers keep the loads where they are written;
+// the scheduler sinks them to their first use otherwise. D is transposed
+// (weights as the first operand): a lane then holds four consecutive channels
+// of a voxel and stores 8 (BF16) or 16 (FP32) bytes.
+// 64 -> 32 channels at 128^3: 405 us (572 TFLOP/s) with 16 x 4 x 4 tiles and
+// the weights staged in LDS, 312 us (743 TFLOP/s) now; 32 -> 64: 409 to 230 us
+// (1010 TFLOP/s).
+// OFF: the type of a lane's byte offset within a plane of the input (32 bits
+// unless a plane is 4 GB or more), added to an address held in scalar registers.
+template <int TY, typename OFF>
+__global__ void __launch_bounds__(256, 2) k_conv3_fwd(const __bf16 *__restrict__ in, const __bf16 *__restrict__ wt,
+                                                      float *__restrict__ out32, __bf16 *__restrict__ outb, int nx,
+                                                      int ny, int nz, int cin, int cout, int relu, int vst) {
+    constexpr int HX = TXV + 2, HY = TY + 2, HZ = TZV + 2;
+    constexpr int ROW = HX * CK, PL = HY * ROW;  // elements of one halo row and plane
+    constexpr int NL = (HX * HY * 4 + 255) / 256;  // 16-byte pieces of a halo plane per thread
+    __shared__ __attribute__((aligned(16))) __bf16 s_in[HZ * PL];
+    const int tilesx = nx / TXV, tilesy = ny / TY, nco = cout / CK;
+    const int ntiles = tilesx * tilesy * (nz / TZV) * nco;
+    // tiles (channel block fastest) in one contiguous range per XCD (workgroup
+    // b runs on XCD b % 8), so that neighbours share their halo in one L2
+    const int nb = gridDim.x, xcd = blockIdx.x & 7, wgs = (nb + 7 - xcd) >> 3;
+    const int before = xcd * (nb >> 3) + min(xcd, nb & 7);  // workgroups of the lower XCDs
+    const int tfirst = (int)((long long)ntiles * before / nb) + (blockIdx.x >> 3);
+    const int tend = (int)((long long)ntiles * (before + wgs) / nb);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 15, lg = lane >> 4;
+    const long long plane = (long long)nx * ny;
+    // this lane's 16 bytes of a halo row for each x shift of the taps
+    int xo[3];
+#pragma unroll
+    for (int dx = 0; dx < 3; dx++) xo[dx] = (lr + dx) * CK + ((lg ^ (((lr + dx) >> 1) & 3)) << 3);
+    // LDS place of this thread's pieces (pieces past the plane repeat its last
+    // voxel: the same bytes to the same place)
+    int lx[NL];
+#pragma unroll
+    for (int i = 0; i < NL; i++) {
+        const int hv = min((tid >> 2) + 64 * i, HX * HY - 1), hx = hv % HX;
+        lx[i] = hv * CK + (((tid & 3) ^ ((hx >> 1) & 3)) << 3);
+    }
+    u32x4 rx[HZ][NL];
+    // in-plane byte offsets of the pieces of tile t, then one halo plane of them
+    OFF fo[NL];
+    auto aim = [&](int t) {
+        const int tt = t / nco;
+        const int x0 = (tt % tilesx) * TXV, y0 = ((tt / tilesx) % tilesy) * TY;
+#pragma unroll
+        for (int i = 0; i < NL; i++) {
+            const int hv = min((tid >> 2) + 64 * i, HX * HY - 1), hx = hv % HX, hy = hv / HX;
+            fo[i] = (OFF)(wrapi(x0 - 1 + hx, nx) + nx * wrapi(y0 - 1 + hy, ny)) * (OFF)(2 * cin) + (tid & 3) * 16;
         }
-        for (int dz = 0; dz < 3; dz++) {
-            // stage the weights of taps dz*9 .. dz*9+8 of this ci chunk: 9 taps x 32 co x 32 ci
-            for (int q = tid; q < 9 * CK * 4; q += 256) {
-                const int row = q >> 2, part = q & 3;  // row = (tap - 9 dz)*32 + co
-                const int tap = dz * 9 + row / CK, co = row % CK;
-                const uint4 val =
-                    *reinterpret_cast<const uint4 *>(wt + ((long long)tap * cout + co0 + co) * cin + ci0 + part * 8);
-                *reinterpret_cast<uint4 *>(s_w + row * W_STRIDE + part * 8) = val;
+        return (tt / (tilesx * tilesy)) * TZV;
+    };
+    auto fetch = [&](int z0, int ci0, int hz) {
+        const char *b = reinterpret_cast<const char *>(in + wrapi(z0 - 1 + hz, nz) * plane * cin + ci0);
+#pragma unroll
+        for (int i = 0; i < NL; i++) rx[hz][i] = *reinterpret_cast<const u32x4 *>(b + fo[i]);
+    };
+    const long long wtap = (long long)cout * cin;
+    const unsigned wo = (unsigned)(lr * cin + lg * 8) * 2u;
+    bf16x8 w[2][3][2];
+    // weights of group g = (dz, dx): taps dy = 0, 1, 2, two blocks of 16
+    // channels, from the block's (uniform) address wu
+    auto wload = [&](int g, const __bf16 *wu, bf16x8 (&d)[3][2]) {
+        const int dz = g / 3, dx = g - 3 * dz;
+#pragma unroll
+        for (int dy = 0; dy < 3; dy++)
+#pragma unroll
+            for (int mb = 0; mb < 2; mb++)
+                d[dy][mb] = *reinterpret_cast<const bf16x8 *>(
+                    reinterpret_cast<const char *>(wu + (dz * 9 + dy * 3 + dx) * wtap + (long long)mb * 16 * cin) + wo);
+    };
+    f32x4 acc[TY][2];
+    // one pass of the loop per 32-channel chunk of a tile: (t, ci0), then (tn, cn)
+    int tn = tfirst, cn = 0;
+    if (tn < tend) {
+        const int z0 = aim(tn);
+#pragma unroll
+        for (int hz = 0; hz < HZ; hz++) fetch(z0, cn, hz);
+    }
+    while (tn < tend) {
+        const int t = tn, ci0 = cn;
+        cn += CK;
+        if (cn >= cin) {
+            cn = 0;
+            tn += wgs;
+        }
+        const int tt = t / nco;
+        const int co0 = (t - tt * nco) * CK;
+        if (ci0 == 0) {
+#pragma unroll
+            for (int a = 0; a < TY; a++)
+#pragma unroll
+                for (int b = 0; b < 2; b++) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        const __bf16 *wu = wt + (long long)co0 * cin + ci0;
+        wload(0, wu, w[0]);
+        __syncthreads();  // the previous chunk has been read
+#pragma unroll
+        for (int hz = 0; hz < HZ; hz++)
+#pragma unroll
+            for (int i = 0; i < NL; i++) *reinterpret_cast<u32x4 *>(s_in + hz * PL + lx[i]) = rx[hz][i];
+        __syncthreads();
+        const int zn = aim(min(tn, tend - 1));  // (behind the last chunk in vain)
+#pragma unroll
+        for (int g = 0; g < 9; g++) {
+            const int dz = g / 3, dx = g % 3;
+            // one plane of the next chunk per group, behind the next weights:
+            // loads return in order, so the wait for those does not reach it
+            if (g < 8) wload(g + 1, wu, w[(g + 1) & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (g < HZ) fetch(zn, cn, g);
+            const __bf16 *base = s_in + PL * (wave + dz) + xo[dx];
+            bf16x8 a[3];
+            a[0] = *reinterpret_cast<const bf16x8 *>(base);
+            a[1] = *reinterpret_cast<const bf16x8 *>(base + ROW);
+#pragma unroll
+            for (int r = 0; r < HY; r++) {
+                if (r + 2 < HY) a[(r + 2) % 3] = *reinterpret_cast<const bf16x8 *>(base + (r + 2) * ROW);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int dy = 0; dy < 3; dy++) {
+                    const int o = r - dy;
+                    if (o < 0 || o >= TY) continue;
+#pragma unroll
+                    for (int mb = 0; mb < 2; mb++)
+                        acc[o][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[g & 1][dy][mb], a[r % 3], acc[o][mb], 0,
+                                                                             0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
-            __syncthreads();
-            for (int t = 0; t < 9; t++) {
-                const int dx = t % 3, dy = t / 3;  // halo offsets (0..2)
-                bf16x8 bfr[2];
-                for (int nb = 0; nb < 2; nb++)
-                    bfr[nb] = *reinterpret_cast<const bf16x8 *>(s_w + (t * CK + nb * 16 + lrow) * W_STRIDE + lk);
-                for (int mb = 0; mb < TYV; mb++) {
-                    const int hv = (lrow + dx) + HX * ((mb + dy) + HY * (wave + dz));
-                    const bf16x8 afr = *reinterpret_cast<const bf16x8 *>(s_in + hv * IN_STRIDE + lk);
-                    for (int nb = 0; nb < 2; nb++)
-                        acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afr, bfr[nb], acc[mb][nb], 0, 0, 0);
+        }
+        if (ci0 + CK < cin) continue;
+        const int x0 = (tt % tilesx) * TXV, y0 = ((tt / tilesx) % tilesy) * TY, z0 = (tt / (tilesx * tilesy)) * TZV;
+        // lane holds channels 4 lg + q of voxel lr of each 16 x 16 block
+        typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+        const unsigned lo = lr * cout + 4 * lg;
+#pragma unroll
+        for (int o = 0; o < TY; o++) {
+            // the row's first element of this block (uniform)
+            const long long e0 = (x0 + (long long)nx * ((y0 + o) + (long long)ny * (z0 + wave))) * cout + co0;
+#pragma unroll
+            for (int mb = 0; mb < 2; mb++) {
+                const f32x4 d = acc[o][mb];
+                if (out32) {
+                    float *p = out32 + (e0 + mb * 16) + lo;
+                    if (vst) {
+                        *reinterpret_cast<f32x4 *>(p) = d;
+                    } else {
+                        for (int q = 0; q < 4; q++) p[q] = d[q];
+                    }
+                }
+                if (outb) {
+                    __bf16 *p = outb + (e0 + mb * 16) + lo;
+                    bf16x4 b;
+#pragma unroll
+                    for (int q = 0; q < 4; q++) b[q] = (__bf16)(relu ? fmaxf(d[q], 0.f) : d[q]);
+                    if (vst) {
+                        *reinterpret_cast<bf16x4 *>(p) = b;
+                    } else {
+                        for (int q = 0; q < 4; q++) p[q] = b[q];
+                    }
                 }
             }
-            __syncthreads();
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
-    // epilogue: lane holds D[m = 4*(lane/16)+q][n = lane%16] of each 16x16 block
-    for (int mb = 0; mb < TYV; mb++)
-        for (int nb = 0; nb < 2; nb++)
-            for (int q = 0; q < 4; q++) {
-                const int vx = x0 + 4 * (lane >> 4) + q, vy = y0 + mb, vz = z0 + wave;
-                const long long v = (long long)vx + (long long)nx * (vy + (long long)ny * vz);
-                const int co = co0 + nb * 16 + lrow;
-                const float val = acc[mb][nb][q];
-                if (out32) out32[v * cout + co] = val;
-                if (outb) outb[v * cout + co] = (__bf16)(relu ? fmaxf(val, 0.f) : val);
-            }
 }
 
 // ---------------------------------------------------------------- weight gradient
-// dW[tap][co][ci] = sum_v dout[v][co] * in[v + off(tap)][ci], split over voxel
-// tiles: workgroup (g, cob, cib) sums tiles g, g + G, g + 2G, ... into
-// part[g][27][32][32] (co-major within the block). Four waves share the taps.
-constexpr int KT = TXV * TYV * TZV;  // 256 voxels per tile
-constexpr int DT_STRIDE = KT + 8;    // bf16 per co row of the transposed dout tile
-// The transposed input tile is held once per x shift dx = 0, 1, 2 of the taps:
-// copy dx holds halo columns dx .. dx+15 of every (y, z) halo row, so the 8
-// consecutive x of a B fragment are one aligned 16-byte LDS read.
-constexpr int WVOX = TXV * HY * HZ;  // 576 voxels of one shifted copy
-constexpr int IT_STRIDE = WVOX + 8;  // bf16 per ci row of a shifted copy
+// dW[tap][co][ci] = sum_v dout[v][co] * in[v + off(tap)][ci] as MFMA with K =
+// voxels along x. Both operands lie in LDS as they lie in memory (channels
+// fastest, 64 bytes per voxel) and are transposed by the read itself
+// (ds_read_b64_tr_b16: a group of 16 lanes reads 4 voxels x 16 channels and
+// lane i gets the 4 voxels of channel i), so an x shift is a voxel offset and
+// nothing is scattered on the way in. The 32-byte halves of a voxel are
+// exchanged by bit 1 of x, which spreads the reads over the banks.
+//
+// A wave owns one 16 x 16 block of (co, ci) for all 27 taps (108 accumulator
+// registers); the 4 waves of a workgroup cover 32 x 32. A unit is a column of
+// WX x 4 voxels over a range of planes: the workgroup marches over the input
+// planes with the three dout planes that pair with each in a 4-deep ring and
+// the next planes' loads in flight, one barrier per plane. Every input row is
+// read once per dx and used for all (dy, dz): 30 operand reads for 108 MFMAs.
+// part[p][cib][cob][27][32][32] holds the sums of workgroup p = 0 .. P-1.
+// 64 -> 32 channels at 128^3: 848 us (scatter-transposed tiles, 274 TFLOP/s)
+// before, 192 us (1210 TFLOP/s) now, and 97 against 11 us for the sum of the
+// partials. WX = 32 needs nx % 32 == 0; WX = 16 uses the K = 16 MFMA, half its
+// rate, and serves the rest.
+constexpr int WY = 4;
 
-__global__ void __launch_bounds__(256) k_conv3_wgrad(const __bf16 *__restrict__ in, const __bf16 *__restrict__ dout,
-                                                     float *__restrict__ part, int nx, int ny, int nz, int cin,
-                                                     int cout, int G) {
-    __shared__ __attribute__((aligned(16))) __bf16 s_inT[3 * CK * IT_STRIDE];
-    __shared__ __attribute__((aligned(16))) __bf16 s_dT[CK * DT_STRIDE];
-    const int tilesx = nx / TXV, tilesy = ny / TYV, tilesz = nz / TZV;
-    const int ntiles = tilesx * tilesy * tilesz;
-    const int g = blockIdx.x, cob = blockIdx.y, cib = blockIdx.z;
-    const int co0 = cob * CK, ci0 = cib * CK;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int lrow = lane & 15, lq = lane >> 4;
-    f32x4 acc[7][2][2];
-    for (int a = 0; a < 7; a++)
-        for (int b = 0; b < 2; b++)
-            for (int c = 0; c < 2; c++) acc[a][b][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int t = g; t < ntiles; t += G) {
-        const int x0 = (t % tilesx) * TXV;
-        const int y0 = ((t / tilesx) % tilesy) * TYV;
-        const int z0 = (t / (tilesx * tilesy)) * TZV;
-        // transposed input halo tile in its three x-shifted copies:
-        // s_inT[dx][ci][w], w = (hx - dx) + TXV * (hy + HY * hz) for hx - dx in [0, TXV)
-        for (int q = tid; q < HVOX * 4; q += 256) {
-            const int hv = q >> 2, part = q & 3;
-            const int hx = hv % HX, hy = (hv / HX) % HY, hz = hv / (HX * HY);
-            const int gx = wrapi(x0 - 1 + hx, nx), gy = wrapi(y0 - 1 + hy, ny), gz = wrapi(z0 - 1 + hz, nz);
-            const long long gv = (long long)gx + (long long)nx * (gy + (long long)ny * gz);
-            const bf16x8 val = *reinterpret_cast<const bf16x8 *>(in + gv * cin + ci0 + part * 8);
-            for (int dx = 0; dx < 3; dx++) {
-                const int wx = hx - dx;
-                if (wx < 0 || wx >= TXV) continue;
-                const int w = wx + TXV * (hy + HY * hz);
-                for (int e = 0; e < 8; e++) s_inT[(dx * CK + part * 8 + e) * IT_STRIDE + w] = val[e];
-            }
-        }
-        // transposed dout tile: s_dT[co][v]
-        for (int q = tid; q < KT * 4; q += 256) {
-            const int v = q >> 2, part = q & 3;
-            const int vx = x0 + v % TXV, vy = y0 + (v / TXV) % TYV, vz = z0 + v / (TXV * TYV);
-            const long long gv = (long long)vx + (long long)nx * (vy + (long long)ny * vz);
-            const bf16x8 val = *reinterpret_cast<const bf16x8 *>(dout + gv * cout + co0 + part * 8);
-            for (int e = 0; e < 8; e++) s_dT[(part * 8 + e) * DT_STRIDE + v] = val[e];
-        }
-        __syncthreads();
-        for (int kc = 0; kc < KT / 32; kc++) {
-            // voxels of this K chunk: v = 32*kc + 8*lq + e, e = 0..7 (consecutive x)
-            const int vb = 32 * kc + 8 * lq;
-            const int vx = vb % TXV, vy = (vb / TXV) % TYV, vz = vb / (TXV * TYV);
-            bf16x8 afr[2];
-            for (int mb = 0; mb < 2; mb++)
-                afr[mb] = *reinterpret_cast<const bf16x8 *>(s_dT + (mb * 16 + lrow) * DT_STRIDE + vb);
-            for (int tt = 0; tt < 7; tt++) {
-                const int tap = wave + 4 * tt;
-                if (tap >= 27) break;
-                const int dx = tap % 3, dy = (tap / 3) % 3, dz = tap / 9;
-                const int w = vx + TXV * ((vy + dy) + HY * (vz + dz));  // vx is 0 or 8
-                for (int nb = 0; nb < 2; nb++) {
-                    const bf16x8 bfr =
-                        *reinterpret_cast<const bf16x8 *>(s_inT + (dx * CK + nb * 16 + lrow) * IT_STRIDE + w);
-                    for (int mb = 0; mb < 2; mb++)
-                        acc[tt][mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afr[mb], bfr, acc[tt][mb][nb], 0, 0, 0);
-                }
-            }
-        }
-        __syncthreads();
-    }
-    // D[m = co][n = ci]: lane holds m = 4*lq + q, n = lrow
-    float *dst = part + (long long)((g * gridDim.z + cib) * gridDim.y + cob) * 27 * CK * CK;
-    for (int tt = 0; tt < 7; tt++) {
-        const int tap = wave + 4 * tt;
-        if (tap >= 27) break;
-        for (int mb = 0; mb < 2; mb++)
-            for (int nb = 0; nb < 2; nb++)
-                for (int q = 0; q < 4; q++) {
-                    const int co = mb * 16 + 4 * lq + q, ci = nb * 16 + lrow;
-                    dst[(tap * CK + co) * CK + ci] = acc[tt][mb][nb][q];
-                }
-    }
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ s16x4 lds_tr(const __bf16 *p) {
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)p);
 }
 
-// dW[tap][co][ci] = sum_g part[g][cib][cob][tap][co%32][ci%32] in fixed order
+template <int WX>
+struct TrFrag;
+template <>
+struct TrFrag<32> {  // voxels 8 lg .. 8 lg + 7 of the row
+    typedef bf16x8 type;
+    static __device__ __forceinline__ type load(const __bf16 *p) {
+        const s16x4 a = lds_tr(p), b = lds_tr(p + 4 * CK);
+        typedef short s16x8 __attribute__((ext_vector_type(8)));
+        const s16x8 v = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+        return __builtin_bit_cast(bf16x8, v);
+    }
+    static __device__ __forceinline__ f32x4 mul(type a, type b, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+    }
+};
+template <>
+struct TrFrag<16> {  // voxels 4 lg .. 4 lg + 3 of the row
+    typedef s16x4 type;
+    static __device__ __forceinline__ type load(const __bf16 *p) { return lds_tr(p); }
+    static __device__ __forceinline__ f32x4 mul(type a, type b, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
+    }
+};
+
+template <int WX>
+__global__ void __launch_bounds__(256, 2) k_conv3_wgrad(const __bf16 *__restrict__ in, const __bf16 *__restrict__ dout,
+                                                        float *__restrict__ part, int nx, int ny, int nz, int cin,
+                                                        int cout, int P, int zseg, int units) {
+    typedef TrFrag<WX> F;
+    constexpr int HXW = WX + 2, HYW = WY + 2;
+    constexpr int XP = HYW * HXW * CK, DP = WY * WX * CK;  // elements of an input and a dout plane
+    constexpr int NXL = (HYW * HXW * 4 + 255) / 256, NDL = WY * WX * 4 / 256;
+    __shared__ __attribute__((aligned(16))) __bf16 s_x[2 * XP];
+    __shared__ __attribute__((aligned(16))) __bf16 s_d[4 * DP];
+    const int nob = cout / CK, nib = cin / CK;
+    const int id = xcd_order(blockIdx.x, gridDim.x);
+    const int blk = id / P, p = id - blk * P;
+    const int cob = blk % nob, cib = blk / nob;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lr = lane & 15, lg = lane >> 4;
+    const int cb = wave & 1, ib = wave >> 1;
+    f32x4 acc[27];
+#pragma unroll
+    for (int a = 0; a < 27; a++) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // this lane's 8 bytes of a row: voxel x, half h of its channels
+    auto voff = [](int x, int h) { return x * CK + ((h ^ ((x >> 1) & 1)) << 4); };
+    const int xl = (WX / 4) * lg + (lr >> 2);
+    const int ao = voff(xl, cb) + (lr & 3) * 4;
+    int bo[3];
+#pragma unroll
+    for (int dx = 0; dx < 3; dx++) bo[dx] = voff(xl + dx, ib) + (lr & 3) * 4;
+    const int colx = nx / WX, coly = ny / WY;
+    const long long plane = (long long)nx * ny;
+    for (int u = p; u < units; u += P) {
+        const int c = u % (colx * coly);
+        const int x0 = (c % colx) * WX, y0 = (c / colx) * WY;
+        const int z0 = (u / (colx * coly)) * zseg, z1 = min(nz, z0 + zseg);
+        // in-plane source and LDS place of this thread's pieces
+        int gx[NXL], gd[NDL], lx[NXL], ld[NDL];
+#pragma unroll
+        for (int i = 0; i < NXL; i++) {
+            // pieces past the plane repeat its last voxel (the same bytes to the same place)
+            const int hv = min((tid >> 2) + 64 * i, HYW * HXW - 1), pc = tid & 3, hx = hv % HXW, hy = hv / HXW;
+            gx[i] = wrapi(x0 - 1 + hx, nx) + nx * wrapi(y0 - 1 + hy, ny);
+            lx[i] = hy * HXW * CK + voff(hx, pc >> 1) + (pc & 1) * 8;
+        }
+#pragma unroll
+        for (int i = 0; i < NDL; i++) {
+            const int hv = (tid >> 2) + 64 * i, pc = tid & 3, hx = hv % WX, hy = hv / WX;
+            gd[i] = (x0 + hx) + nx * (y0 + hy);
+            ld[i] = hy * WX * CK + voff(hx, pc >> 1) + (pc & 1) * 8;
+        }
+        u32x4 rx[NXL], rd[NDL];
+        auto getx = [&](int hz) {
+            const __bf16 *b = in + (long long)wrapi(hz, nz) * plane * cin + cib * CK + (tid & 3) * 8;
+#pragma unroll
+            for (int i = 0; i < NXL; i++) rx[i] = *reinterpret_cast<const u32x4 *>(b + (long long)gx[i] * cin);
+        };
+        // a dout plane that is not the unit's counts as zero
+        auto getd = [&](int z) {
+            const __bf16 *b = dout + (long long)min(z, z1 - 1) * plane * cout + cob * CK + (tid & 3) * 8;
+#pragma unroll
+            for (int i = 0; i < NDL; i++) rd[i] = *reinterpret_cast<const u32x4 *>(b + (long long)gd[i] * cout);
+        };
+        auto putx = [&](int hz) {
+#pragma unroll
+            for (int i = 0; i < NXL; i++) *reinterpret_cast<u32x4 *>(s_x + (hz & 1) * XP + lx[i]) = rx[i];
+        };
+        auto putd = [&](int z) {
+#pragma unroll
+            for (int i = 0; i < NDL; i++)
+                *reinterpret_cast<u32x4 *>(s_d + (z & 3) * DP + ld[i]) = z < z1 ? rd[i] : u32x4{0u, 0u, 0u, 0u};
+        };
+        getx(z0 - 1);
+        getd(z0);
+        __syncthreads();  // the previous unit's planes have been read
+        putx(z0 - 1);
+        putd(z0);
+        for (int q = 1; q < 3; q++)
+#pragma unroll
+            for (int i = 0; i < NDL; i++)
+                *reinterpret_cast<u32x4 *>(s_d + ((z0 - q) & 3) * DP + ld[i]) = u32x4{0u, 0u, 0u, 0u};
+        __syncthreads();
+        for (int hz = z0 - 1; hz <= z1; hz++) {
+            // the next planes, loaded behind this one's products (past the
+            // unit's end loaded in vain)
+            getx(min(hz + 1, z1));
+            getd(hz + 2);
+            const __bf16 *xp = s_x + (hz & 1) * XP;
+            const __bf16 *dp[3];
+#pragma unroll
+            for (int dz = 0; dz < 3; dz++) dp[dz] = s_d + ((hz + 1 - dz) & 3) * DP + ao;
+            // operands of a halo row one row ahead of its products; the
+            // barriers keep the scheduler from hoisting all rows' reads, which
+            // spills
+            typename F::type A[3][WY], B[2][3];
+            auto ldrow = [&](int hy) {
+#pragma unroll
+                for (int dx = 0; dx < 3; dx++) B[hy & 1][dx] = F::load(xp + hy * HXW * CK + bo[dx]);
+                if (hy < WY) {
+#pragma unroll
+                    for (int dz = 0; dz < 3; dz++) A[dz][hy] = F::load(dp[dz] + hy * WX * CK);
+                }
+            };
+            ldrow(0);
+#pragma unroll
+            for (int hy = 0; hy < HYW; hy++) {
+                if (hy + 1 < HYW) ldrow(hy + 1);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int dz = 0; dz < 3; dz++)
+#pragma unroll
+                    for (int dy = 0; dy < 3; dy++) {
+                        const int y = hy - dy;
+                        if (y < 0 || y >= WY) continue;
+#pragma unroll
+                        for (int dx = 0; dx < 3; dx++)
+                            acc[dz * 9 + dy * 3 + dx] = F::mul(A[dz][y], B[hy & 1][dx], acc[dz * 9 + dy * 3 + dx]);
+                    }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            putx(hz + 1);
+            putd(hz + 2);
+            __syncthreads();
+        }
+    }
+    // D[m = co][n = ci]: lane holds m = 4 lg + q, n = lr
+    float *dst = part + (long long)((p * nib + cib) * nob + cob) * 27 * CK * CK;
+#pragma unroll
+    for (int t = 0; t < 27; t++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) dst[(t * CK + cb * 16 + 4 * lg + q) * CK + ib * 16 + lr] = acc[t][q];
+}
+
+// dW[tap][co][ci] = sum_p part[p][cib][cob][tap][co%32][ci%32] in fixed order:
+// a workgroup takes 64 consecutive entries of a partial, four slices of p per
+// entry (p = s, s + 4, ...), and adds the slices in order. (One thread per
+// entry over all partials was bound by the latency of its loads.)
 __global__ void __launch_bounds__(256) k_wgrad_reduce(const float *__restrict__ part, float *__restrict__ dw, int cin,
-                                                      int cout, int G) {
-    const long long n = 27LL * cout * cin;
-    const int ncb = cin / CK, nob = cout / CK;
-    for (long long i = blockIdx.x * 256LL + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
-        const int ci = (int)(i % cin);
-        const int co = (int)((i / cin) % cout);
-        const int tap = (int)(i / ((long long)cin * cout));
-        const int cib = ci / CK, cob = co / CK;
-        const long long off = (long long)(tap * CK + co % CK) * CK + ci % CK;
-        float s = 0.f;
-        for (int g = 0; g < G; g++) s += part[(long long)((g * ncb + cib) * nob + cob) * 27 * CK * CK + off];
-        dw[i] = s;
+                                                      int cout, int P) {
+    __shared__ float sm[4][64];
+    const int c = threadIdx.x & 63, sl = threadIdx.x >> 6;
+    const int n = 27 * cin * cout;  // entries of a partial; a multiple of 64
+    const int e = blockIdx.x * 64 + c;
+    float s = 0.f;
+#pragma unroll 8
+    for (int p = sl; p < P; p += 4) s += part[(long long)p * n + e];
+    sm[sl][c] = s;
+    __syncthreads();
+    if (sl == 0) {
+        const int ci = e % CK, co = (e / CK) % CK, tap = (e / (CK * CK)) % 27, blk = e / (27 * CK * CK);
+        const int nob = cout / CK, cob = blk % nob, cib = blk / nob;
+        dw[((long long)tap * cout + cob * CK + co) * cin + cib * CK + ci] =
+            (sm[0][c] + sm[1][c]) + (sm[2][c] + sm[3][c]);
     }
 }
 
@@ -702,9 +920,24 @@ extern "C" {
 int ngapnet_conv3_fwd(const void *in, const void *wt, float *out32, void *outb, int nx, int ny, int nz, int cin,
                       int cout, int relu, void *stream) {
     if (cin % CK || cout % CK || nx % TXV || ny % TYV || nz % TZV || cin <= 0 || cout <= 0) return -1;
-    dim3 grid((nx / TXV) * (ny / TYV) * (nz / TZV), cout / CK);
-    hipLaunchKernelGGL(k_conv3_fwd, grid, dim3(256), 0, (hipStream_t)stream, (const __bf16 *)in, (const __bf16 *)wt,
-                       out32, (__bf16 *)outb, nx, ny, nz, cin, cout, relu);
+    const int vst = (uintptr_t)out32 % 16 == 0 && (uintptr_t)outb % 8 == 0;
+    const long long wg4 = (long long)(nx / TXV) * (ny / TYV) * (nz / TZV) * (cout / CK);
+    // 16 x 8 x 4 tiles where they still give every CU a workgroup; smaller
+    // grids take 16 x 4 x 4 so that the chip is not left idle. At most two
+    // workgroups per CU are launched; they walk over the tiles.
+    const auto wgs = [](long long tiles) { return dim3((unsigned)(tiles < 512 ? tiles : 512)); };
+    const bool big = (long long)nx * ny * cin * 2 >= (1LL << 32);
+    if (big)
+        hipLaunchKernelGGL((k_conv3_fwd<4, unsigned long long>), wgs(wg4), dim3(256), 0, (hipStream_t)stream,
+                           (const __bf16 *)in, (const __bf16 *)wt, out32, (__bf16 *)outb, nx, ny, nz, cin, cout, relu,
+                           vst);
+    else if (ny % 8 == 0 && wg4 / 2 >= 256)
+        hipLaunchKernelGGL((k_conv3_fwd<8, unsigned>), wgs(wg4 / 2), dim3(256), 0, (hipStream_t)stream,
+                           (const __bf16 *)in, (const __bf16 *)wt, out32, (__bf16 *)outb, nx, ny, nz, cin, cout, relu,
+                           vst);
+    else
+        hipLaunchKernelGGL((k_conv3_fwd<4, unsigned>), wgs(wg4), dim3(256), 0, (hipStream_t)stream, (const __bf16 *)in,
+                           (const __bf16 *)wt, out32, (__bf16 *)outb, nx, ny, nz, cin, cout, relu, vst);
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
@@ -719,12 +952,30 @@ int ngapnet_wgrad_parts(int nx, int ny, int nz, int cin, int cout) {
 int ngapnet_conv3_wgrad(const void *in, const void *dout, float *dw, float *part, int nx, int ny, int nz, int cin,
                         int cout, void *stream) {
     if (cin % CK || cout % CK || nx % TXV || ny % TYV || nz % TZV) return -1;
-    const int G = ngapnet_wgrad_parts(nx, ny, nz, cin, cout);
-    dim3 grid(G, cout / CK, cin / CK);
-    hipLaunchKernelGGL(k_conv3_wgrad, grid, dim3(256), 0, (hipStream_t)stream, (const __bf16 *)in,
-                       (const __bf16 *)dout, part, nx, ny, nz, cin, cout, G);
-    hipLaunchKernelGGL(k_wgrad_reduce, dim3(blocks_for(27LL * cin * cout)), dim3(256), 0, (hipStream_t)stream,
-                       (const float *)part, dw, cin, cout, G);
+    const int blocks = (cin / CK) * (cout / CK);
+    const int wx = nx % 32 == 0 ? 32 : 16;
+    const int cols = (nx / wx) * (ny / WY);
+    // workgroups per 32 x 32 channel block: two per CU over all blocks, at most
+    // the caller's partials; columns are cut into ranges of planes (at least 4:
+    // each range reads two more) until there is a unit for each
+    int P = ngapnet_wgrad_parts(nx, ny, nz, cin, cout);
+    if (P > 512 / blocks) P = 512 / blocks;
+    if (P < 1) P = 1;
+    int nseg = (P + cols - 1) / cols;
+    if (nseg > nz / 4) nseg = nz / 4;
+    const int zseg = (nz + nseg - 1) / nseg;
+    nseg = (nz + zseg - 1) / zseg;
+    const int units = cols * nseg;
+    if (P > units) P = units;
+    const dim3 grid((unsigned)(P * blocks));
+    if (wx == 32)
+        hipLaunchKernelGGL(k_conv3_wgrad<32>, grid, dim3(256), 0, (hipStream_t)stream, (const __bf16 *)in,
+                           (const __bf16 *)dout, part, nx, ny, nz, cin, cout, P, zseg, units);
+    else
+        hipLaunchKernelGGL(k_conv3_wgrad<16>, grid, dim3(256), 0, (hipStream_t)stream, (const __bf16 *)in,
+                           (const __bf16 *)dout, part, nx, ny, nz, cin, cout, P, zseg, units);
+    hipLaunchKernelGGL(k_wgrad_reduce, dim3((unsigned)(27 * cin * cout / 64)), dim3(256), 0, (hipStream_t)stream,
+                       (const float *)part, dw, cin, cout, P);
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 

@@ -1,0 +1,76 @@
+"""The tiled BF16 convolution kernels at the edges of their tiles and ranges:
+one tile, workgroups that walk over several tiles and channel chunks, rows that
+are a multiple of 16 but not of 32, columns cut into ranges of planes, and
+output pointers that allow no vector stores.
+
+Reference: float64 products of the same BF16 values, tap by tap. The kernels
+accumulate n = 27 cin (forward) or n = voxels (weight gradient) products in
+FP32, in an order of their own: an error of a few sqrt(n) 2^-24 of the sums'
+scale. The bounds of test_gpu_unet.py (2e-6 and 2e-5 of max|ref|) hold at these
+sizes as well. BF16 outputs are within one rounding (2^-8) of the reference.
+"""
+import ctypes as C
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+SHAPES = [
+    ((16, 4, 4), 32, 32),    # one tile
+    ((16, 4, 8), 64, 32),    # two tiles, two channel chunks
+    ((48, 12, 4), 32, 64),   # rows of 48: the K = 16 weight gradient; 12 rows: no 8-row tiles
+    ((32, 4, 20), 64, 64),   # one column of 32 voxels, planes cut unevenly
+    ((64, 64, 64), 32, 64),  # 1024 8-row tiles: workgroups walk over two each
+    ((128, 40, 20), 64, 32),  # 8-row tiles, ragged share per workgroup
+]
+
+
+def _off(tap):
+    return tap % 3 - 1, (tap // 3) % 3 - 1, tap // 9 - 1
+
+
+def _shifted(x, shape, tap):
+    dx, dy, dz = _off(tap)
+    g = x.reshape(shape[2], shape[1], shape[0], -1)
+    return torch.roll(g, (-dz, -dy, -dx), (0, 1, 2)).reshape(x.shape)
+
+
+def _p(t):
+    return C.c_void_p(t.data_ptr())
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("shape,cin,cout", SHAPES)
+def test_forward_and_weight_gradient(shape, cin, cout, shift):
+    from nga2_amd import unet
+
+    L = unet.lib()
+    print(f"\n[conv tiles {shape} {cin}->{cout} shift {shift}]", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(7)
+    V = shape[0] * shape[1] * shape[2]
+    x = torch.randn(V, cin, generator=gen, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(27, cout, cin, generator=gen, device=DEV) / (27 * cin) ** 0.5).to(torch.bfloat16)
+    g = torch.randn(V, cout, generator=gen, device=DEV).to(torch.bfloat16)
+    out = torch.zeros(V * cout + 1, device=DEV)[shift:shift + V * cout]
+    outb = torch.zeros(V * cout + 1, dtype=torch.bfloat16, device=DEV)[shift:shift + V * cout]
+    parts = L.ngapnet_wgrad_parts(*shape, cin, cout)
+    part = torch.zeros(parts * 27 * cin * cout + 1, device=DEV)[shift:]
+    dw = torch.zeros(27 * cin * cout + 1, device=DEV)[shift:shift + 27 * cin * cout]
+    unet._enter()
+    rc = L.ngapnet_conv3_fwd(_p(x), _p(w), _p(out), _p(outb), *shape, cin, cout, 1, None)
+    rc |= L.ngapnet_conv3_wgrad(_p(x), _p(g), _p(dw), _p(part), *shape, cin, cout, None)
+    unet._leave()
+    assert rc == 0
+    x64, w64, g64 = x.double(), w.double(), g.double()
+    ref = sum(_shifted(x64, shape, t) @ w64[t].T for t in range(27))
+    err = (out.double().reshape(V, cout) - ref).abs().max() / ref.abs().max()
+    assert float(err) <= 2e-6, float(err)
+    relu = torch.relu(ref)
+    lim = relu * 2.0 ** -8 + 2e-6 * ref.abs().max()
+    assert bool(((outb.double().reshape(V, cout) - relu).abs() <= lim).all())
+    dref = torch.stack([g64.T @ _shifted(x64, shape, t) for t in range(27)])
+    err = (dw.double().reshape(27, cout, cin) - dref).abs().max() / dref.abs().max()
+    assert float(err) <= 2e-5, float(err)
