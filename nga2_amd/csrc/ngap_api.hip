@@ -1038,14 +1038,18 @@ void coarse_solve(ngap_t *h, const T *f, T *v) {
     }
 }
 
-// First level of the small-level bottom (k_bottom), or nlev when the
-// bottom is not used: it needs the dense coarsest solve, at least one
-// smoothing level below the fine level, and at most BOT_MAX_LEVELS levels.
+// First level of the small-level bottom (k_bottom) in precision T, or nlev when
+// the bottom is not used: it needs the dense coarsest solve, at least one
+// smoothing level below the fine level, at most BOT_MAX_LEVELS levels, and
+// levels that fit it.
+template <typename T>
 int bottom_start(const ngap_t *h) {
     const int nl = h->nlev;
     if (!h->coarse_dense || nl < 3) return nl;
+    std::vector<Geo> g;
+    for (const Level &L : h->lev) g.push_back(L.g);
     int lb = nl - 1;
-    while (lb - 1 >= 1 && h->lev[lb - 1].g.N <= BOT_MAX_CELLS && nl - (lb - 1) <= BOT_MAX_LEVELS) lb--;
+    while (lb - 1 >= 1 && nl - (lb - 1) <= BOT_MAX_LEVELS && bottom_fits<T>(&g[lb - 1], nl - (lb - 1))) lb--;
     return lb <= nl - 2 ? lb : nl;
 }
 
@@ -1059,7 +1063,7 @@ void launch_bottom_levels(ngap_t *h, int lb) {
     for (int q = 0; q < a.nlev; q++) {
         Level &L = h->lev[lb + q];
         LevelData<T> &D = data<T>(L);
-        a.L[q] = BotLevel<T>{L.g, L.cdir, L.relax ? 1 : 0, D.c, D.a0, D.a1, D.a2, D.pm, D.pp, D.f, D.v, D.w};
+        a.L[q] = BotLevel<T>{L.g, BotDir{L.cdir}, L.relax ? 1 : 0, D.c, D.a0, D.a1, D.a2, D.pm, D.pp, D.f, D.v, 0.0f, 0.0f};
     }
     launch_bottom<T>(h->stream, a);
 }
@@ -1094,7 +1098,7 @@ void vcycle(ngap_t *h, const T *f0, T *v0) {
         if (L.g.N < PAIR_MIN_CELLS || npre < 2) return npre;
         return 1 + (npre - 2) / 2 + ((npre - 2) & 1);
     };
-    const int lb = bottom_start(h);
+    const int lb = bottom_start<T>(h);
     const int top = lb < nl ? lb : nl - 1;  // first level below the per-level loop
     std::vector<T *> pre(nl);
     for (int l = 0; l < top; l++) {

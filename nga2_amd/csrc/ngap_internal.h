@@ -50,23 +50,32 @@ int apply_blocks(const Geo &g, int &kc);
 
 // The small levels of a V-cycle in one workgroup (see k_bottom).
 constexpr int BOT_MAX_LEVELS = 16;
-constexpr long long BOT_MAX_CELLS = 1024;
+// Coarsening to the next level: the direction, and along it the cells and
+// strides of this level and the next (all but d set by launch_bottom).
+struct BotDir {
+    int d, nf, nc, per, sf, sc;
+};
 template <typename T>
 struct BotLevel {
     Geo g;
-    int cdir;   // coarsening direction to the next level
+    BotDir dir;
     int relax;  // 0: skipped level (no smoothing, see set_relax)
     const T *c, *a0, *a1, *a2;
     const T *pm, *pp;  // transfer weights from the finer level (coarse-indexed)
-    T *f, *v, *w;
+    T *f, *v;
+    float ih, i1;  // 1 / ceil(n0 / 2), 1 / n1 (set by launch_bottom)
 };
 template <typename T>
 struct BotArgs {
     int nlev;  // levels lb..lb+nlev-1, the last one solved by the dense inverse
     int npre, npost;
+    int cap;  // entries of the kernel's work arrays (set by launch_bottom)
     const double *Ainv;
     BotLevel<T> L[BOT_MAX_LEVELS];
 };
+// whether the n levels g[0] .. g[n-1] (the last the coarsest) fit the bottom kernel
+template <typename T>
+bool bottom_fits(const Geo *g, int n);
 template <typename T>
 void launch_bottom(hipStream_t s, const BotArgs<T> &a);
 void launch_strength(hipStream_t s, const Geo &g, const double *a0, const double *a1, const double *a2, double *part,

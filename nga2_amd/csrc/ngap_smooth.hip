@@ -1106,23 +1106,38 @@ __global__ void __launch_bounds__(256) k_dense_t(int n, const double *__restrict
 }
 
 // ------------------------------------------------------------------ bottom of the V-cycle
-// The levels of at most BOT_MAX_CELLS cells, from the pre-smoothing of the
-// first of them through the dense coarsest solve back to its post-smoothing,
-// in one workgroup of 1024 threads with a barrier between phases. On these
-// levels every launch of the per-level kernels costs a few microseconds of
-// latency for a few thousand cells of work. Sweeps are in place (each colour
-// reads only the other colour, so this equals the out-of-place sweeps of the
-// large levels), and every sum keeps the order of the per-level kernels.
-// A phase gives each thread at most one cell (BOT_MAX_CELLS = 1024): out of
-// range threads are clamped to the last cell and do not store, so the code
-// has no branch around the loads. (Taking 4096-cell levels here, with four
-// cells per thread, measured slower than their per-level kernels.) Global
-// memory written before a barrier is read after it by other threads of the
-// same workgroup (one CU, one L1), which __syncthreads orders.
+// The small levels (bottom_fits() below), from the pre-smoothing of the first
+// of them through the dense coarsest solve back to its post-smoothing, in one
+// workgroup of 1024 threads with a barrier between phases. On these levels
+// every launch of the per-level kernels costs a few microseconds of latency for
+// a few thousand cells of work. Every sum keeps the order of the per-level
+// kernels, and sweeps in place equal the out-of-place ones (each colour reads
+// only the other colour), so the results are theirs bit for bit.
+//
+// A phase is bound by latency: its loads, the chain of six multiply-adds, the
+// division, the barrier. So everything is in LDS: at the start the coefficients
+// of all levels are copied there with all loads in flight, and the right-hand
+// sides and iterates of the way down stay there for the way up. A thread owns
+// one cell of either colour of a level and holds its coefficients, right-hand
+// side and neighbour places in registers through the level's phases. The
+// iterate in work is stored by colour: with h = ceil(n0 / 2) cells of a colour
+// per row and H = h n1 n2, cell (x, j, k) of colour c = (x + j + k) & 1 lies at
+// c H + (k n1 + j) h + x / 2: all neighbours are of the other colour, each
+// phase reads one half with unit stride, and no lane idles on the other
+// colour's cells.
+// Beyond the latency a level costs its instructions (16 waves on one CU: 16
+// cycles each), so red and black cell share one set of indices, waves without
+// cells wait at the barriers, and the code is kept small (a workgroup passes
+// through it once: versions with several cells per thread for levels up to 8192
+// cells spent 150 us and more fetching instructions).
+// FP32 V(2,2), the levels of 1024 cells and below of the 256^3 channel: 56 us
+// with indices and global loads in every phase; 35 us now with the level of 2048
+// cells too, which took 29 us in nine launches. FP64 V(1,1), 64^3 periodic: 29
+// against 22 us.
 namespace {
 
 constexpr int BT_THREADS = 1024;
-constexpr int BT_CPT = 1;  // cells per thread and phase
+constexpr int BT_LDS = 158 * 1024;  // bytes of LDS the kernel uses
 
 // q = p / d for 0 <= p < 2^24 from a float reciprocal, corrected to exact
 __device__ __forceinline__ int bt_div(int p, int d, float inv) {
@@ -1132,228 +1147,328 @@ __device__ __forceinline__ int bt_div(int p, int d, float inv) {
     return q;
 }
 
-__device__ __forceinline__ void bt_ijk(const Geo &g, int p, int &i, int &j, int &k) {
-    const float i0 = 1.0f / (float)g.n0, i1 = 1.0f / (float)g.n1;
-    const int r = bt_div(p, g.n0, i0);
-    i = p - r * g.n0;
-    k = bt_div(r, g.n1, i1);
-    j = r - k * g.n1;
+// place of a cell in a level's colour-split iterate, h = ceil(n0 / 2), H = h n1 n2
+__device__ __forceinline__ int bt_at(const Geo &g, int h, int H, int x, int j, int k) {
+    return ((x + j + k) & 1) * H + (k * g.n1 + j) * h + (x >> 1);
 }
 
-// neighbour offsets of cell p (0 where there is no neighbour; `has` bits
-// -x +x -y +y -z +z)
-struct BtNb {
-    int xm, xp, ym, yp, zm, zp;
-    int has;
+// One cell of a thread: diagonal, right-hand side, the couplings to its six
+// neighbours (0 where there is none), their places in the other colour's half,
+// its own place, its x and its flat index (-1: no cell)
+template <typename T>
+struct BtCell {
+    T c, f, a[6];
+    int nb[6];
+    int at, x, p;
 };
 
-__device__ __forceinline__ BtNb bt_nb(const Geo &g, int p, int &parity) {
-    int i, j, k;
-    bt_ijk(g, p, i, j, k);
-    parity = (i + j + k) & 1;
-    const int n0 = g.n0, plane = g.n0 * g.n1;
-    const int im = nbm(i, g.n0, g.p0), ip = nbp(i, g.n0, g.p0);
-    const int jm = nbm(j, g.n1, g.p1), jp = nbp(j, g.n1, g.p1);
-    const int km = nbm(k, g.n2, g.p2), kp = nbp(k, g.n2, g.p2);
-    BtNb b;
-    b.has = (im >= 0) | ((ip >= 0) << 1) | ((jm >= 0) << 2) | ((jp >= 0) << 3) | ((km >= 0) << 4) | ((kp >= 0) << 5);
-    b.xm = im >= 0 ? p - i + im : p;
-    b.xp = ip >= 0 ? p - i + ip : p;
-    b.ym = jm >= 0 ? p + (jm - j) * n0 : p;
-    b.yp = jp >= 0 ? p + (jp - j) * n0 : p;
-    b.zm = km >= 0 ? p + (km - k) * plane : p;
-    b.zp = kp >= 0 ? p + (kp - k) * plane : p;
-    return b;
+// A thread's red and black cell of a level: x = 2 u and 2 u + 1 of row (j, k)
+template <typename T>
+struct BtPair {
+    BtCell<T> r, b;
+    int j, k;
+};
+
+// q = the place in a colour (q < H), A = c, a0, a1, a2 (N entries each)
+template <typename T>
+__device__ __forceinline__ void bt_pair(const Geo &g, float ih, float i1, int q, const T *A, BtPair<T> &S) {
+    const int h = (g.n0 + 1) >> 1, H = h * g.n1 * g.n2, N = (int)g.N, plane = g.n0 * g.n1;
+    const int row = bt_div(q, h, ih), u = q - row * h;
+    const int k = bt_div(row, g.n1, i1), j = row - k * g.n1;
+    const int e = (j + k) & 1;  // colour of the even cell
+    const bool odd = 2 * u + 1 < g.n0;
+    const int p0 = row * g.n0 + 2 * u, p1 = odd ? p0 + 1 : p0;  // a missing odd cell loads the even one's
+    const T *a0 = A + N, *a1 = A + 2 * N, *a2 = A + 3 * N;
+    // x: even - left uL, right u; odd - left u, right uR (place in the row, -1: none)
+    const int uL = u > 0 ? u - 1 : (g.p0 ? h - 1 : -1);
+    const int uR = 2 * u + 2 < g.n0 ? u + 1 : (g.p0 && g.n0 > 1 ? 0 : -1);
+    const int q0 = row * h;
+    // y, z: the same place of the neighbouring rows; a direction of one cell has
+    // no neighbour (a periodic one couples to itself with 0)
+    const int jm = j > 0 ? -1 : (g.p1 ? g.n1 - 1 : 0), jp = j < g.n1 - 1 ? 1 : (g.p1 ? 1 - g.n1 : 0);
+    const int km = k > 0 ? -1 : (g.p2 ? g.n2 - 1 : 0), kp = k < g.n2 - 1 ? 1 : (g.p2 ? 1 - g.n2 : 0);
+    const int hn = h * g.n1;
+    const int qym = q + jm * h, qyp = q + jp * h, qzm = q + km * hn, qzp = q + kp * hn;
+    const T z = T(0);
+    const T cE = A[p0], cO = A[p1];
+    const T xE = a0[p0], xO = a0[p1], xN = a0[row * g.n0 + (uR >= 0 ? 2 * uR : 0)];
+    const T ymE = a1[p0], ymO = a1[p1], ypE = a1[p0 + jp * g.n0], ypO = a1[p1 + jp * g.n0];
+    const T zmE = a2[p0], zmO = a2[p1], zpE = a2[p0 + kp * plane], zpO = a2[p1 + kp * plane];
+    auto fill = [=](BtCell<T> &C, int col, bool even) {
+        const int o = (col ^ 1) * H;
+        const bool hl = even ? uL >= 0 : true, hr = even ? odd : uR >= 0;
+        C.c = even ? cE : cO;
+        C.a[0] = hl ? (even ? xE : xO) : z;
+        C.a[1] = hr ? (even ? xO : xN) : z;
+        C.a[2] = jm ? (even ? ymE : ymO) : z;
+        C.a[3] = jp ? (even ? ypE : ypO) : z;
+        C.a[4] = km ? (even ? zmE : zmO) : z;
+        C.a[5] = kp ? (even ? zpE : zpO) : z;
+        C.nb[0] = o + q0 + (hl ? (even ? uL : u) : u);
+        C.nb[1] = o + q0 + (hr ? (even ? u : uR) : u);
+        C.nb[2] = o + qym;
+        C.nb[3] = o + qyp;
+        C.nb[4] = o + qzm;
+        C.nb[5] = o + qzp;
+        C.at = col * H + q;
+        C.x = 2 * u + (even ? 0 : 1);
+        C.p = even ? p0 : (odd ? p1 : -1);
+    };
+    fill(S.r, 0, e == 0);
+    fill(S.b, 1, e == 1);
+    S.j = j;
+    S.k = k;
 }
 
-// in-place red/black phase: cells of `colour` get (f - sum a v_nb) / c
-// (zero: the iterate is zero, so the cell gets f / c)
+// (f - sum a v_nb) / c in the order and with the roundings of the per-level
+// sweeps: each multiply-add rounds once, explicitly, as the conditional ones
+// there do (a plain c v + a v' may be fused either way)
 template <typename T>
-__device__ void bt_colour(const BotLevel<T> &L, T *v, int colour, bool zero) {
-    const int N = (int)L.g.N;
-    for (int base = 0; base < N; base += BT_THREADS * BT_CPT) {
-        T res[BT_CPT];
-        int pp[BT_CPT];
-        bool st[BT_CPT];
+__device__ __forceinline__ void bt_relax(const BtCell<T> &S, T *V) {
+#pragma clang fp contract(off)
+    T v[6];
 #pragma unroll
-        for (int m = 0; m < BT_CPT; m++) {
-            const int q = base + m * BT_THREADS + (int)threadIdx.x;
-            const int p = q < N ? q : N - 1;
-            int par;
-            const BtNb b = bt_nb(L.g, p, par);
-            T sum = L.f[p];
-            if (!zero) {
-                const T vxm = v[b.xm], vxp = v[b.xp], vym = v[b.ym], vyp = v[b.yp], vzm = v[b.zm], vzp = v[b.zp];
-                const T axm = L.a0[p], axp = L.a0[b.xp], aym = L.a1[p], ayp = L.a1[b.yp], azm = L.a2[p],
-                        azp = L.a2[b.zp];
-                if (b.has & 1) sum -= axm * vxm;
-                if (b.has & 2) sum -= axp * vxp;
-                if (b.has & 4) sum -= aym * vym;
-                if (b.has & 8) sum -= ayp * vyp;
-                if (b.has & 16) sum -= azm * vzm;
-                if (b.has & 32) sum -= azp * vzp;
-            }
-            res[m] = sum / L.c[p];
-            pp[m] = p;
-            st[m] = q < N && par == colour;
-        }
+    for (int d = 0; d < 6; d++) v[d] = V[S.nb[d]];
+    T sum = S.f;
 #pragma unroll
-        for (int m = 0; m < BT_CPT; m++)
-            if (st[m]) v[pp[m]] = res[m];
-    }
+    for (int d = 0; d < 6; d++) sum = fma_t(-S.a[d], v[d], sum);
+    if (S.p >= 0) V[S.at] = sum / S.c;
 }
 
-// w = f - A v
+// R[p] = f - A v, and the iterate to K[p]
 template <typename T>
-__device__ void bt_resid(const BotLevel<T> &L, const T *v, T *w) {
-    const int N = (int)L.g.N;
-    for (int base = 0; base < N; base += BT_THREADS * BT_CPT) {
+__device__ __forceinline__ void bt_resid(const BtCell<T> &S, const T *V, T *R, T *K) {
+#pragma clang fp contract(off)
+    if (S.p < 0) return;
+    const T vc = V[S.at];
+    T t = S.c * vc;
 #pragma unroll
-        for (int m = 0; m < BT_CPT; m++) {
-            const int q = base + m * BT_THREADS + (int)threadIdx.x;
-            const int p = q < N ? q : N - 1;
-            int par;
-            const BtNb b = bt_nb(L.g, p, par);
-            const T vc = v[p], vxm = v[b.xm], vxp = v[b.xp], vym = v[b.ym], vyp = v[b.yp], vzm = v[b.zm],
-                    vzp = v[b.zp];
-            T t = L.c[p] * vc;
-            if (b.has & 1) t += L.a0[p] * vxm;
-            if (b.has & 2) t += L.a0[b.xp] * vxp;
-            if (b.has & 4) t += L.a1[p] * vym;
-            if (b.has & 8) t += L.a1[b.yp] * vyp;
-            if (b.has & 16) t += L.a2[p] * vzm;
-            if (b.has & 32) t += L.a2[b.zp] * vzp;
-            if (q < N) w[p] = L.f[p] - t;
-        }
-    }
+    for (int d = 0; d < 6; d++) t = fma_t(S.a[d], V[S.nb[d]], t);
+    R[S.p] = S.f - t;
+    K[S.p] = vc;
 }
 
-__device__ __forceinline__ int bt_dim(const Geo &g, int d) { return d == 0 ? g.n0 : (d == 1 ? g.n1 : g.n2); }
-__device__ __forceinline__ int bt_per(const Geo &g, int d) { return d == 0 ? g.p0 : (d == 1 ? g.p1 : g.p2); }
-
-// fc = P^T r along direction d (as k_gather_t)
+// (P^T r) at coarse cell (I, J, K) along direction d (as k_gather_t), r by flat index
 template <typename T>
-__device__ void bt_gather(const Geo &F, const Geo &C, int d, const T *r, const T *__restrict__ pm,
-                          const T *__restrict__ pp, T *fc) {
-    const int N = (int)C.N;
-    for (int base = 0; base < N; base += BT_THREADS * BT_CPT) {
-#pragma unroll
-        for (int m = 0; m < BT_CPT; m++) {
-            const int q = base + m * BT_THREADS + (int)threadIdx.x;
-            const int pc = q < N ? q : N - 1;
-            int I, J, K;
-            bt_ijk(C, pc, I, J, K);
-            const int i = d == 0 ? 2 * I : I, j = d == 1 ? 2 * J : J, k = d == 2 ? 2 * K : K;
-            const int e = d == 0 ? i : (d == 1 ? j : k);
-            const int nd = bt_dim(F, d), per = bt_per(F, d);
-            const int stride = d == 0 ? 1 : (d == 1 ? F.n0 : F.n0 * F.n1);
-            const int pf = (k * F.n1 + j) * F.n0 + i;
-            const int l = nbm(e, nd, per);
-            const bool hasr = e + 1 < nd;
-            const int Jd = d == 0 ? I : (d == 1 ? J : K);
-            const int jl = l >= 0 ? nbm(Jd, bt_dim(C, d), bt_per(C, d)) : Jd;
-            const int pl = d == 0 ? (K * C.n1 + J) * C.n0 + jl
-                                  : (d == 1 ? (K * C.n1 + jl) * C.n0 + I : (jl * C.n1 + J) * C.n0 + I);
-            const T r0 = r[pf], rr = r[hasr ? pf + stride : pf], rl = r[l >= 0 ? pf + (l - e) * stride : pf];
-            const T wm = pm[pc], wp = pp[pl];
-            T s = r0;
-            if (hasr) s += wm * rr;
-            if (l >= 0) s += wp * rl;
-            if (q < N) fc[pc] = s;
-        }
-    }
+__device__ __forceinline__ T bt_gather(const Geo &F, const Geo &C, const BotDir &D, const T *R, const T *pm,
+                                       const T *pp, int I, int J, int K) {
+#pragma clang fp contract(off)
+    const int d = D.d, nd = D.nf, per = D.per, nc = D.nc, sf = D.sf, sc = D.sc;
+    const int Jd = d == 0 ? I : (d == 1 ? J : K);
+    const int pc = (K * C.n1 + J) * C.n0 + I;
+    const int pf = ((d == 2 ? 2 * K : K) * F.n1 + (d == 1 ? 2 * J : J)) * F.n0 + (d == 0 ? 2 * I : I);
+    const bool hasl = Jd > 0 || per, hasr = 2 * Jd + 1 < nd;
+    const int pl = Jd > 0 ? pf - sf : (per ? pf + (nd - 1) * sf : pf);
+    const int wl = Jd > 0 ? pc - sc : (per ? pc + (nc - 1) * sc : pc);
+    const T wm = pm[pc], wp = pp[wl], rr = R[hasr ? pf + sf : pf], rl = R[pl];
+    T s = R[pf];
+    if (hasr) s = fma_t(wm, rr, s);
+    if (hasl) s = fma_t(wp, rl, s);
+    return s;
 }
 
-// v += P vc along direction d (as k_prolong_t)
+// (P vc) at fine cell (i, j, k) along direction d (as k_prolong_t), vc stored by colour
 template <typename T>
-__device__ void bt_prolong(const Geo &F, const Geo &C, int d, const T *__restrict__ pm, const T *__restrict__ pp,
-                           const T *vc, T *v) {
-    const int N = (int)F.N;
-    for (int base = 0; base < N; base += BT_THREADS * BT_CPT) {
-#pragma unroll
-        for (int m = 0; m < BT_CPT; m++) {
-            const int q = base + m * BT_THREADS + (int)threadIdx.x;
-            const int p = q < N ? q : N - 1;
-            int i, j, k;
-            bt_ijk(F, p, i, j, k);
-            const int fd = d == 0 ? i : (d == 1 ? j : k);
-            const int Jd = fd >> 1;
-            const int I = d == 0 ? Jd : i, J = d == 1 ? Jd : j, K = d == 2 ? Jd : k;
-            const int pl = (K * C.n1 + J) * C.n0 + I;
-            const int jr = nbp(Jd, bt_dim(C, d), bt_per(C, d));
-            const bool odd = fd & 1, hasr = jr >= 0;
-            const int pr = !hasr ? pl
-                                 : (d == 0 ? (K * C.n1 + J) * C.n0 + jr
-                                           : (d == 1 ? (K * C.n1 + jr) * C.n0 + I : (jr * C.n1 + J) * C.n0 + I));
-            const T v0 = v[p], c0 = vc[pl], c1 = vc[pr], wm = pm[pl], wp = pp[pl];
-            T add;
-            if (!odd) {
-                add = c0;
-            } else {
-                add = wm * c0;
-                if (hasr) add += wp * c1;
-            }
-            if (q < N) v[p] = v0 + add;
-        }
-    }
+__device__ __forceinline__ T bt_prolong(const Geo &C, const BotDir &D, const T *pm, const T *pp, const T *vc, int i,
+                                        int j, int k) {
+#pragma clang fp contract(off)
+    const int h = (C.n0 + 1) >> 1, H = h * C.n1 * C.n2, d = D.d, nc = D.nc, per = D.per;
+    const int fd = d == 0 ? i : (d == 1 ? j : k), Jd = fd >> 1;
+    const int I = d == 0 ? Jd : i, J = d == 1 ? Jd : j, K = d == 2 ? Jd : k;
+    const bool hasr = Jd < nc - 1 || per;
+    const int jr = Jd < nc - 1 ? Jd + 1 : (per ? 0 : Jd);
+    const int pl = (K * C.n1 + J) * C.n0 + I;
+    const T x0 = vc[bt_at(C, h, H, I, J, K)];
+    const T x1 = vc[bt_at(C, h, H, d == 0 ? jr : I, d == 1 ? jr : J, d == 2 ? jr : K)];
+    const T m = pm[pl] * x0, q = fma_t(pp[pl], x1, m);
+    return (fd & 1) ? (hasr ? q : m) : x0;
 }
 
 template <typename T>
 __global__ void __launch_bounds__(BT_THREADS) k_bottom(BotArgs<T> a) {
-    const int nl = a.nlev;
+    constexpr int E = BT_LDS / (int)sizeof(T);
+    __shared__ T M[E];
+    const int nl = a.nlev, npre = a.npre, npost = a.npost, cap = a.cap, tid = (int)threadIdx.x;
+    // two iterates by colour and the residual (cap entries each), then per level
+    // c, a0, a1, a2, pm, pp, f and the iterate of the way down (N entries each)
+    T *R = M + 2 * cap;
+#pragma unroll 1
+    for (int l = 0, base = 3 * cap; l < nl; l++) {
+        const int N = (int)a.L[l].g.N;
+        T *d = M + base;
+        const T *s0 = a.L[l].c, *s1 = a.L[l].a0, *s2 = a.L[l].a1, *s3 = a.L[l].a2, *s4 = a.L[l].pm, *s5 = a.L[l].pp;
+        for (int q = tid; q < N; q += BT_THREADS) {
+            const T v0 = s0[q], v1 = s1[q], v2 = s2[q], v3 = s3[q], v4 = s4[q], v5 = s5[q];
+            d[q] = v0;
+            d[N + q] = v1;
+            d[2 * N + q] = v2;
+            d[3 * N + q] = v3;
+            d[4 * N + q] = v4;
+            d[5 * N + q] = v5;
+            if (l == 0) d[6 * N + q] = a.L[0].f[q];
+        }
+        base += 8 * N;
+    }
+    __syncthreads();
+    BtPair<T> S;  // this thread's cells
     // down: pre-smoothing, residual, restriction
+    int base = 3 * cap;
+#pragma unroll 1
     for (int l = 0; l < nl - 1; l++) {
-        const BotLevel<T> &L = a.L[l];
-        if (!L.relax) {
+        const Geo g = a.L[l].g;
+        const int N = (int)g.N, relax = a.L[l].relax, H = ((g.n0 + 1) >> 1) * g.n1 * g.n2;
+        const bool act = tid < H;
+        T *D = M + base, *fs = D + 6 * N;
+        if (act) {
+            bt_pair<T>(g, a.L[l].ih, a.L[l].i1, tid, D, S);
+            if (l > 0) {
+                const Geo F = a.L[l - 1].g;
+                const BotDir d = a.L[l - 1].dir;
+                if (S.r.p >= 0) fs[S.r.p] = bt_gather<T>(F, g, d, R, D + 4 * N, D + 5 * N, S.r.x, S.j, S.k);
+                if (S.b.p >= 0) fs[S.b.p] = bt_gather<T>(F, g, d, R, D + 4 * N, D + 5 * N, S.b.x, S.j, S.k);
+            }
+            S.r.f = fs[S.r.p >= 0 ? S.r.p : 0];
+            S.b.f = fs[S.b.p >= 0 ? S.b.p : 0];
+        }
+        if (!relax) {
             // skipped level: v = 0 (the prolongation adds to it), f restricted as it is
-            for (int p = threadIdx.x; p < (int)L.g.N; p += BT_THREADS) L.v[p] = T(0);
-            bt_gather<T>(L.g, a.L[l + 1].g, L.cdir, L.f, a.L[l + 1].pm, a.L[l + 1].pp, a.L[l + 1].f);
-            __syncthreads();
-            continue;
+            __syncthreads();  // R has been read
+            if (act) {
+                if (S.r.p >= 0) R[S.r.p] = S.r.f;
+                if (S.b.p >= 0) R[S.b.p] = S.b.f;
+            }
+        } else {
+            // the first colour from zero; places without a cell are read with a zero coupling
+            if (act) {
+                M[S.r.at] = S.r.p >= 0 ? S.r.f / S.r.c : T(0);
+                M[S.b.at] = T(0);
+            }
+#pragma unroll 1
+            for (int sw = 0;;) {
+                __syncthreads();
+                if (act) bt_relax<T>(S.b, M);
+                __syncthreads();
+                if (++sw == npre) break;
+                if (act) bt_relax<T>(S.r, M);
+            }
+            if (act) {
+                bt_resid<T>(S.r, M, R, D + 7 * N);
+                bt_resid<T>(S.b, M, R, D + 7 * N);
+            }
         }
-        for (int sw = 0; sw < a.npre; sw++) {
-            bt_colour<T>(L, L.v, 0, sw == 0);
-            __syncthreads();
-            bt_colour<T>(L, L.v, 1, false);
-            __syncthreads();
-        }
-        bt_resid<T>(L, L.v, L.w);
         __syncthreads();
-        bt_gather<T>(L.g, a.L[l + 1].g, L.cdir, L.w, a.L[l + 1].pm, a.L[l + 1].pp, a.L[l + 1].f);
-        __syncthreads();
+        base += 8 * N;
     }
     // coarsest: v = Ainv f, one wavefront per row (lane-strided columns, as k_dense_t)
     {
-        const BotLevel<T> &C = a.L[nl - 1];
-        const int n = (int)C.g.N;
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        const Geo C = a.L[nl - 1].g, F = a.L[nl - 2].g;
+        const BotDir d = a.L[nl - 2].dir;
+        const int n = (int)C.N, h = (C.n0 + 1) >> 1, H = h * C.n1 * C.n2;
+        const double *Ainv = a.Ainv;
+        T *D = M + base, *fc = D + 6 * n, *vc = D + 7 * n;
+        int i = 0, j = 0, k = 0;
+        if (tid < n) {
+            const int r = bt_div(tid, C.n0, 1.0f / (float)C.n0);
+            i = tid - r * C.n0;
+            k = bt_div(r, C.n1, a.L[nl - 1].i1);
+            j = r - k * C.n1;
+            fc[tid] = bt_gather<T>(F, C, d, R, D + 4 * n, D + 5 * n, i, j, k);
+        }
+        __syncthreads();
+        const int lane = tid & 63, wave = tid >> 6;
+#pragma unroll 4
         for (int row = wave; row < n; row += BT_THREADS / 64) {
             double s = 0.0;
-            for (int jj = lane; jj < n; jj += 64) s += a.Ainv[(long long)row * n + jj] * (double)C.f[jj];
+            for (int jj = lane; jj < n; jj += 64) s += Ainv[(long long)row * n + jj] * (double)fc[jj];
             s = wave_sum(s);
-            if (lane == 0) C.v[row] = (T)s;
+            if (lane == 0) vc[row] = (T)s;
         }
+        __syncthreads();
+        if (tid < n) M[bt_at(C, h, H, i, j, k)] = vc[tid];
         __syncthreads();
     }
     // up: prolongation and post-smoothing (the other colour first)
+    int vb = 0;
+#pragma unroll 1
     for (int l = nl - 2; l >= 0; l--) {
-        const BotLevel<T> &L = a.L[l];
-        bt_prolong<T>(L.g, a.L[l + 1].g, L.cdir, a.L[l + 1].pm, a.L[l + 1].pp, a.L[l + 1].v, L.v);
+        const Geo g = a.L[l].g, C = a.L[l + 1].g;
+        const int N = (int)g.N, NC = (int)C.N, relax = a.L[l].relax;
+        const BotDir d = a.L[l].dir;
+        const bool act = tid < ((g.n0 + 1) >> 1) * g.n1 * g.n2;
+        const T *pm = M + base + 4 * NC, *pp = M + base + 5 * NC, *vc = M + vb * cap;
+        base -= 8 * N;
+        const T *D = M + base;
+        vb ^= 1;
+        T *V = M + vb * cap;
+        if (act) {
+            bt_pair<T>(g, a.L[l].ih, a.L[l].i1, tid, D, S);
+            const int rp = S.r.p >= 0 ? S.r.p : 0, bp = S.b.p >= 0 ? S.b.p : 0;
+            S.r.f = D[6 * N + rp];
+            S.b.f = D[6 * N + bp];
+            // a missing cell's x is the last one's here
+            const int rx = S.r.p >= 0 ? S.r.x : S.b.x, bx = S.b.p >= 0 ? S.b.x : S.r.x;
+            const T rv = (relax ? D[7 * N + rp] : T(0)) + bt_prolong<T>(C, d, pm, pp, vc, rx, S.j, S.k);
+            const T bv = (relax ? D[7 * N + bp] : T(0)) + bt_prolong<T>(C, d, pm, pp, vc, bx, S.j, S.k);
+            V[S.r.at] = S.r.p >= 0 ? rv : T(0);
+            V[S.b.at] = S.b.p >= 0 ? bv : T(0);
+        }
         __syncthreads();
-        if (!L.relax) continue;
-        for (int sw = 0; sw < a.npost; sw++) {
-            bt_colour<T>(L, L.v, 1, false);
-            __syncthreads();
-            bt_colour<T>(L, L.v, 0, false);
-            __syncthreads();
+        if (relax)
+#pragma unroll 1
+            for (int sw = 0; sw < npost; sw++) {
+                if (act) bt_relax<T>(S.b, V);
+                __syncthreads();
+                if (act) bt_relax<T>(S.r, V);
+                __syncthreads();
+            }
+        if (l == 0 && act) {
+            T *vout = a.L[0].v;
+            if (S.r.p >= 0) vout[S.r.p] = V[S.r.at];
+            if (S.b.p >= 0) vout[S.b.p] = V[S.b.at];
         }
     }
 }
 
 }  // namespace
 
+// Whether levels of these shapes, first to coarsest, are the bottom kernel's:
+// one cell of a colour per thread, and all arrays in its LDS (2048 FP32 or 1024
+// FP64 cells in the first level of a halving sequence).
+static long long bottom_places(const Geo &g) { return 2LL * ((g.n0 + 1) / 2) * g.n1 * g.n2; }
+
 template <typename T>
-void launch_bottom(hipStream_t s, const BotArgs<T> &a) {
+bool bottom_fits(const Geo *g, int n) {
+    long long cap = 0, cells = 0;
+    for (int l = 0; l < n; l++) {
+        const long long q = bottom_places(g[l]);
+        if (l < n - 1 && q > 2 * BT_THREADS) return false;
+        cap = std::max(cap, q);
+        cells += g[l].N;
+    }
+    return (3 * cap + 8 * cells) * (long long)sizeof(T) <= BT_LDS;
+}
+
+template <typename T>
+void launch_bottom(hipStream_t s, const BotArgs<T> &args) {
+    BotArgs<T> a = args;
+    long long cap = 0;
+    for (int l = 0; l < a.nlev; l++) {
+        const Geo &g = a.L[l].g;
+        cap = std::max(cap, bottom_places(g));
+        a.L[l].ih = 1.0f / (float)((g.n0 + 1) / 2);
+        a.L[l].i1 = 1.0f / (float)g.n1;
+        if (l + 1 < a.nlev) {
+            const Geo &c = a.L[l + 1].g;
+            BotDir &D = a.L[l].dir;
+            const int nf[3] = {g.n0, g.n1, g.n2}, nc[3] = {c.n0, c.n1, c.n2}, per[3] = {g.p0, g.p1, g.p2};
+            D.nf = nf[D.d];
+            D.nc = nc[D.d];
+            D.per = per[D.d];
+            D.sf = D.d == 0 ? 1 : (D.d == 1 ? g.n0 : g.n0 * g.n1);
+            D.sc = D.d == 0 ? 1 : (D.d == 1 ? c.n0 : c.n0 * c.n1);
+        }
+    }
+    a.cap = (int)cap;
     hipLaunchKernelGGL(k_bottom<T>, dim3(1), dim3(BT_THREADS), 0, s, a);
 }
 
@@ -1669,6 +1784,8 @@ void launch_dense(hipStream_t s, int n, const double *Ainv, const Tin *f, Tout *
     hipLaunchKernelGGL((k_dense_t<Tin, Tout>), dim3((n + 3) / 4), dim3(256), 0, s, n, Ainv, f, v);
 }
 
+template bool bottom_fits<double>(const Geo *, int);
+template bool bottom_fits<float>(const Geo *, int);
 template void launch_bottom<double>(hipStream_t, const BotArgs<double> &);
 template void launch_bottom<float>(hipStream_t, const BotArgs<float> &);
 
