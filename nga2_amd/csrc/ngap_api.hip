@@ -24,7 +24,7 @@ namespace {
 
 // ---------------------------------------------------------------- scalar slots
 enum { S_RR = 0, S_BB, S_RHO, S_ALPHA, S_BETA, S_PQ, S_RHO0, S_BAD, S_RRT, S_ASYM, S_STR0, S_STR1, S_STR2, S_CSING,
-       S_CBAD, S_NSCAL };
+       S_CBAD, S_XNZ, S_NSCAL };
 constexpr int NSCAL_ALLOC = 16;
 // device and pinned host scalars, then 4 int flags in the same allocation
 constexpr size_t SCAL_BYTES = sizeof(double) * NSCAL_ALLOC + sizeof(int) * 4;
@@ -43,11 +43,12 @@ __device__ __forceinline__ long long gidx(const Ghost &h, int i, int j, int k) {
     return (long long)(i + h.oi) + h.nxo * ((long long)(j + h.oj) + h.nyo * (long long)(k + h.ok));
 }
 
+// cell coordinates of p < 2^31 (setup rejects larger grids), in 32 bits
 __device__ __forceinline__ void decomp0(const Geo &g, long long p, int &i, int &j, int &k) {
-    i = (int)(p % g.n0);
-    long long r = p / g.n0;
-    j = (int)(r % g.n1);
-    k = (int)(r / g.n1);
+    const unsigned q = (unsigned)p, r = q / (unsigned)g.n0;
+    i = (int)(q - r * (unsigned)g.n0);
+    k = (int)(r / (unsigned)g.n1);
+    j = (int)(r - (unsigned)k * (unsigned)g.n1);
 }
 
 __device__ __forceinline__ long long lin0(const Geo &g, int i, int j, int k) {
@@ -153,22 +154,28 @@ __global__ void __launch_bounds__(NT) k_level0(Geo g, Ghost gh, Slots sl, const 
 
 // ---------------------------------------------------------------- solve kernels
 
-// dst = part ? src(ghosted) : 0; counts non-finite values of participating cells
+// dst = part ? src(ghosted) : 0; counts non-finite values of participating
+// cells (p_bad) and values that are not zero (p_nz)
 __global__ void __launch_bounds__(NT) k_gather(Geo g, Ghost gh, const double *__restrict__ src,
                                                const unsigned char *__restrict__ part, double *__restrict__ dst,
-                                               double *__restrict__ p_bad) {
+                                               double *__restrict__ p_bad, double *__restrict__ p_nz) {
     __shared__ double sm[NT / 64];
-    double bad = 0.0;
+    double bad = 0.0, nz = 0.0;
     for (long long p = blockIdx.x * (long long)NT + threadIdx.x; p < g.N; p += (long long)gridDim.x * NT) {
         int i, j, k;
         decomp0(g, p, i, j, k);
         double v = part[p] ? src[gidx(gh, i, j, k)] : 0.0;
         if (!isfinite(v)) bad += 1.0;
+        if (v != 0.0) nz += 1.0;
         dst[p] = v;
     }
     if (p_bad) {
         double b = block_sum(bad, sm);
         if (threadIdx.x == 0) p_bad[blockIdx.x] = b;
+    }
+    if (p_nz) {
+        double b = block_sum(nz, sm);
+        if (threadIdx.x == 0) p_nz[blockIdx.x] = b;
     }
 }
 
@@ -181,36 +188,93 @@ __global__ void __launch_bounds__(NT) k_scatter(Geo g, Ghost gh, const double *_
     }
 }
 
+// The six neighbours of a cell: flat offsets, 0 where there is none (has bit q)
+struct Nb6 {
+    int o[6];
+    int has;
+};
+__device__ __forceinline__ Nb6 nb6(const Geo &g, int i, int j, int k) {
+    const int plane = g.n0 * g.n1;
+    const int ip = nbp(i, g.n0, g.p0), im = nbm(i, g.n0, g.p0);
+    const int jp = nbp(j, g.n1, g.p1), jm = nbm(j, g.n1, g.p1);
+    const int kp = nbp(k, g.n2, g.p2), km = nbm(k, g.n2, g.p2);
+    Nb6 n;
+    n.o[0] = ip >= 0 ? ip - i : 0;
+    n.o[1] = im >= 0 ? im - i : 0;
+    n.o[2] = jp >= 0 ? (jp - j) * g.n0 : 0;
+    n.o[3] = jm >= 0 ? (jm - j) * g.n0 : 0;
+    n.o[4] = kp >= 0 ? (kp - k) * plane : 0;
+    n.o[5] = km >= 0 ? (km - k) * plane : 0;
+    n.has = (ip >= 0) | (im >= 0) << 1 | (jp >= 0) << 2 | (jm >= 0) << 3 | (kp >= 0) << 4 | (km >= 0) << 5;
+    return n;
+}
+
+// The two exact products below are bound by the latency of their loads: a
+// thread works on PU cells of its stride at a time, all loads issued before
+// the first use and none behind a branch.
+constexpr int PU = 2;
+
 // r = b - A x with the exact 7-array operator (identity rows where the
 // centre is 0; couplings out of a non-periodic box ignored); partial ||r||^2.
+// The 7 entries of a cell are adjacent in opr, 56 bytes from cell to cell, so a
+// wave copies the entries of its 64 consecutive cells through LDS with
+// coalesced 8-byte loads. 256^3: 444 us one cell at a time, each lane reading
+// its own entries; 309 us now.
 __global__ void __launch_bounds__(NT) k_exact_resid(Geo g, Ghost gh, Slots sl, const double *__restrict__ opr,
                                                     const double *__restrict__ b, const double *__restrict__ x,
                                                     double *__restrict__ r, double *__restrict__ part) {
     __shared__ double sm[NT / 64];
+    __shared__ double st[PU * NT * OPR_NST];
+    double *w = st + (threadIdx.x & ~63u) * (PU * OPR_NST);  // this wave's entries
+    const int lane = threadIdx.x & 63;
+    const long long stride = (long long)gridDim.x * NT;
     double acc = 0.0;
-    for (long long p = blockIdx.x * (long long)NT + threadIdx.x; p < g.N; p += (long long)gridDim.x * NT) {
-        int i, j, k;
-        decomp0(g, p, i, j, k);
-        const double *A = opr + gidx(gh, i, j, k) * sl.nst;
-        double s;
-        double a0 = A[sl.s[0]];
-        if (!(fabs(a0) > 0.0)) {
-            s = x[p];
-        } else {
-            s = a0 * x[p];
-            int ip = nbp(i, g.n0, g.p0), im = nbm(i, g.n0, g.p0);
-            int jp = nbp(j, g.n1, g.p1), jm = nbm(j, g.n1, g.p1);
-            int kp = nbp(k, g.n2, g.p2), km = nbm(k, g.n2, g.p2);
-            if (ip >= 0) s += A[sl.s[1]] * x[lin0(g, ip, j, k)];
-            if (im >= 0) s += A[sl.s[2]] * x[lin0(g, im, j, k)];
-            if (jp >= 0) s += A[sl.s[3]] * x[lin0(g, i, jp, k)];
-            if (jm >= 0) s += A[sl.s[4]] * x[lin0(g, i, jm, k)];
-            if (kp >= 0) s += A[sl.s[5]] * x[lin0(g, i, j, kp)];
-            if (km >= 0) s += A[sl.s[6]] * x[lin0(g, i, j, km)];
+    for (long long pw = blockIdx.x * (long long)NT + (threadIdx.x & ~63u); pw < g.N; pw += PU * stride) {
+        int p[PU];
+        Nb6 nb[PU];
+        double av[PU][OPR_NST], xv[PU][7], bv[PU];
+#pragma unroll
+        for (int u = 0; u < PU; u++) {
+            const long long q = pw + u * stride + lane;
+            p[u] = q < g.N ? (int)q : (int)g.N - 1;
+            int i, j, k;
+            decomp0(g, p[u], i, j, k);
+            const int gs = (int)gidx(gh, i, j, k);  // ghosted cells fit in 31 bits (checked at setup)
+#pragma unroll
+            for (int m = 0; m < OPR_NST; m++) {
+                const int e = lane + 64 * m, cl = e / OPR_NST, c = e - cl * OPR_NST;
+                av[u][m] = opr[(long long)__shfl(gs, cl, 64) * OPR_NST + c];
+            }
+            nb[u] = nb6(g, i, j, k);
+            xv[u][0] = x[p[u]];
+#pragma unroll
+            for (int d = 0; d < 6; d++) xv[u][d + 1] = x[p[u] + nb[u].o[d]];
+            bv[u] = b[p[u]];
         }
-        double rv = b[p] - s;
-        r[p] = rv;
-        acc += rv * rv;
+        __builtin_amdgcn_wave_barrier();  // the previous cells' entries have been read (one wave: LDS works in order)
+#pragma unroll
+        for (int u = 0; u < PU; u++)
+#pragma unroll
+            for (int m = 0; m < OPR_NST; m++) w[u * 64 * OPR_NST + lane + 64 * m] = av[u][m];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int u = 0; u < PU; u++) {
+            const double *A = w + (u * 64 + lane) * OPR_NST;
+            const double a0 = A[sl.s[0]];
+            double s = a0 * xv[u][0];
+#pragma unroll
+            for (int d = 0; d < 6; d++) {
+                const double t = __builtin_fma(A[sl.s[d + 1]], xv[u][d + 1], s);
+                s = (nb[u].has >> d) & 1 ? t : s;
+            }
+            if (!(fabs(a0) > 0.0)) s = xv[u][0];
+            if (pw + u * stride + lane < g.N) {
+                const double rv = bv[u] - s;
+                r[p[u]] = rv;
+                acc += rv * rv;
+            }
+        }
     }
     double t = block_sum(acc, sm);
     if (threadIdx.x == 0) part[blockIdx.x] = t;
@@ -237,32 +301,45 @@ __global__ void __launch_bounds__(NT) k_soa7(Geo g, Ghost gh, Slots sl, const do
 }
 
 // y = A x, or (b != nullptr) r = b - A x with partial ||r||^2 in part, from the
-// seven-array form; the same sum order as k_exact_resid
+// seven-array form; the same sum order as k_exact_resid. 128^3: 42 us one cell
+// at a time; 33 us now.
 __global__ void __launch_bounds__(NT) k_apply7(Geo g, const double *__restrict__ o7, const double *__restrict__ b,
                                                const double *__restrict__ x, double *__restrict__ y,
                                                double *__restrict__ part) {
     __shared__ double sm[NT / 64];
     double acc = 0.0;
-    const long long N = g.N;
-    for (long long p = blockIdx.x * (long long)NT + threadIdx.x; p < N; p += (long long)gridDim.x * NT) {
-        int i, j, k;
-        decomp0(g, p, i, j, k);
-        double s = o7[p] * x[p];
-        const int ip = nbp(i, g.n0, g.p0), im = nbm(i, g.n0, g.p0);
-        const int jp = nbp(j, g.n1, g.p1), jm = nbm(j, g.n1, g.p1);
-        const int kp = nbp(k, g.n2, g.p2), km = nbm(k, g.n2, g.p2);
-        if (ip >= 0) s += o7[N + p] * x[lin0(g, ip, j, k)];
-        if (im >= 0) s += o7[2 * N + p] * x[lin0(g, im, j, k)];
-        if (jp >= 0) s += o7[3 * N + p] * x[lin0(g, i, jp, k)];
-        if (jm >= 0) s += o7[4 * N + p] * x[lin0(g, i, jm, k)];
-        if (kp >= 0) s += o7[5 * N + p] * x[lin0(g, i, j, kp)];
-        if (km >= 0) s += o7[6 * N + p] * x[lin0(g, i, j, km)];
-        if (b) {
-            const double rv = b[p] - s;
-            y[p] = rv;
-            acc += rv * rv;
-        } else {
-            y[p] = s;
+    const long long N = g.N, stride = (long long)gridDim.x * NT;
+    for (long long p0 = blockIdx.x * (long long)NT + threadIdx.x; p0 < N; p0 += PU * stride) {
+        int p[PU];
+        Nb6 nb[PU];
+        double ov[PU][7], xv[PU][7], bv[PU];
+#pragma unroll
+        for (int u = 0; u < PU; u++) {
+            const long long q = p0 + u * stride;
+            p[u] = q < N ? (int)q : (int)N - 1;
+            int i, j, k;
+            decomp0(g, p[u], i, j, k);
+            nb[u] = nb6(g, i, j, k);
+#pragma unroll
+            for (int d = 0; d < 7; d++) ov[u][d] = o7[d * N + p[u]];
+            xv[u][0] = x[p[u]];
+#pragma unroll
+            for (int d = 0; d < 6; d++) xv[u][d + 1] = x[p[u] + nb[u].o[d]];
+            bv[u] = b ? b[p[u]] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < PU; u++) {
+            double s = ov[u][0] * xv[u][0];
+#pragma unroll
+            for (int d = 0; d < 6; d++) {
+                const double t = __builtin_fma(ov[u][d + 1], xv[u][d + 1], s);
+                s = (nb[u].has >> d) & 1 ? t : s;
+            }
+            if (p0 + u * stride < N) {
+                const double rv = b ? bv[u] - s : s;
+                y[p[u]] = rv;
+                if (b) acc += rv * rv;
+            }
         }
     }
     if (part) {
@@ -617,6 +694,12 @@ __global__ void k_clear_flags(int *flags) {
     if (threadIdx.x == 0) flags[0] = 0;
 }
 
+// workgroups of a streaming kernel without partial sums, `per` cells a thread
+int stream_blocks(long long n, int per) {
+    const long long b = (n + (long long)NT * per - 1) / ((long long)NT * per);
+    return (int)(b < 1 ? 1 : (b > 65536 ? 65536 : b));
+}
+
 double now_ms() {
     return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
@@ -692,6 +775,7 @@ struct ngap_t {
     int fail_alloc = 0;      // > 0: the fail_alloc-th next device allocation fails (ngapt_fail_alloc)
     Staging stg;             // pinned staging of ngap_solve, made on its first call
     int relax_keep = 1;      // levels 0..relax_keep-1 are always smoothed (set_relax)
+    bool x_zero = false;     // the guess of the solve in work is zero (counted with check_finite)
     bool p32 = false;        // p holds FP32 values (the mixed solve's directions), set at each restart
     long long zero_chunks = 0;  // guess chunks of the last ngap_solve found all zero (not copied)
     // the last setup completed with these options; its levels and coarsening
@@ -1683,7 +1767,13 @@ int run_pcg(ngap_t *h) {
     h->st.stage_calls = 0;
     if (stage_pc && (rc = stage_bufs(h))) return rc;
     hipLaunchKernelGGL(k_clear_flags, dim3(1), dim3(64), 0, s, h->flags);
-    exact_residual(h, h->r, S_RR);
+    // from a zero guess (its values and the operator's are known to be finite)
+    // the residual is b, and its norm the sum below: the product with the
+    // exact operator is left out
+    if (h->x_zero)
+        hipLaunchKernelGGL(k_copy, dim3(nb), dim3(NT), 0, s, N, (const double *)h->b, h->r);
+    else
+        exact_residual(h, h->r, S_RR);
     hipLaunchKernelGGL(k_sumsq, dim3(nb), dim3(NT), 0, s, N, (const double *)h->b, h->parts + MAX_PARTS);
     hipLaunchKernelGGL(k_fin_sum, dim3(1), dim3(NT), 0, s, (const double *)(h->parts + MAX_PARTS), nb, h->scal,
                        (int)S_BB);
@@ -1701,7 +1791,7 @@ int run_pcg(ngap_t *h) {
         h->st.status = NGAP_STATUS_CONVERGED;
         return 0;
     }
-    double rel = std::sqrt(h->h_scal[S_RR]) / bn;
+    double rel = std::sqrt(h->h_scal[h->x_zero ? S_BB : S_RR]) / bn;
     const double tol = h->rcvg;
     if (h->stage_fn && (h->stage_flags & NGAP_STAGE_GUESS) && rel > tol && std::isfinite(rel)) {
         if ((rc = guess_stage(h, bn, &rel))) return rc;
@@ -1942,7 +2032,8 @@ int run_gmres(ngap_t *h) {
             double *vj = h->gV + (size_t)j * N, *zj = h->gZ + (size_t)j * N;
             double *w = h->gV + (size_t)(j + 1) * N;
             gmres_precond(h, vj, zj, mixed);
-            hipLaunchKernelGGL(k_apply7, dim3(nb), dim3(NT), 0, s, h->g0, (const double *)h->o7,
+            // (no partial sums: as many workgroups as there is work for)
+            hipLaunchKernelGGL(k_apply7, dim3(stream_blocks(N, PU)), dim3(NT), 0, s, h->g0, (const double *)h->o7,
                                (const double *)nullptr, (const double *)zj, w, (double *)nullptr);
             cgs_pass(h, w, h->gV, j + 1, h->gm, -1);
             cgs_pass(h, w, h->gV, j + 1, h->gm + 64, 128);
@@ -2155,25 +2246,32 @@ int do_solve(ngap_t *h, const double *rhs, double *sol, bool on_device, int *it,
         dsol = h->sol_g;
     }
     const long long N = h->g0.N;
-    const int nb = grid_for(N);
+    // counts are exact in any order, so these take more partial sums than the
+    // solver's reductions (256^3: 100 us with 1024 workgroups, 66 us now)
+    const int nb = std::min(grid_parts(N), 4096);
     hipLaunchKernelGGL(k_gather, dim3(nb), dim3(NT), 0, s, h->g0, h->gh, drhs, (const unsigned char *)h->part, h->b,
-                       h->opts.check_finite ? h->parts : (double *)nullptr);
+                       h->opts.check_finite ? h->parts : (double *)nullptr, (double *)nullptr);
     if (h->opts.check_finite)
         hipLaunchKernelGGL(k_fin_sum, dim3(1), dim3(NT), 0, s, (const double *)h->parts, nb, h->scal, (int)S_BAD);
     hipLaunchKernelGGL(k_gather, dim3(nb), dim3(NT), 0, s, h->g0, h->gh, (const double *)dsol,
-                       (const unsigned char *)h->part, h->x, h->opts.check_finite ? h->parts + MAX_PARTS : nullptr);
+                       (const unsigned char *)h->part, h->x, h->opts.check_finite ? h->parts + MAX_PARTS : nullptr,
+                       h->opts.check_finite ? h->parts + 2 * MAX_PARTS : nullptr);
+    h->x_zero = false;
     if (h->opts.check_finite) {
         hipLaunchKernelGGL(k_fin_sum, dim3(1), dim3(NT), 0, s, (const double *)(h->parts + MAX_PARTS), nb, h->scal,
                            (int)S_RRT);
+        hipLaunchKernelGGL(k_fin_sum, dim3(1), dim3(NT), 0, s, (const double *)(h->parts + 2 * MAX_PARTS), nb, h->scal,
+                           (int)S_XNZ);
         HIPCHK(hipGetLastError());
         int rc = read_scal(h);
         if (rc) return rc;
         if (h->h_scal[S_BAD] > 0.0 || h->h_scal[S_RRT] > 0.0) return NGAP_ERR_NONFINITE;
+        h->x_zero = h->h_scal[S_XNZ] == 0.0;
     }
     HIPCHK(hipGetLastError());
     int rc = h->method == NGAP_GMRES_PFMG ? run_gmres(h) : run_pcg(h);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_scatter, dim3(nb), dim3(NT), 0, s, h->g0, h->gh, (const double *)h->x, dsol);
+    hipLaunchKernelGGL(k_scatter, dim3(stream_blocks(N, 4)), dim3(NT), 0, s, h->g0, h->gh, (const double *)h->x, dsol);
     HIPCHK(hipGetLastError());
     if (!on_device) {
         HIPCHK(hipStreamSynchronize(s));
@@ -2482,9 +2580,9 @@ int ngap_residual_device(ngap_t *h, const double *d_rhs, const double *d_sol, do
     const long long N = h->g0.N;
     const int nb = grid_for(N);
     hipLaunchKernelGGL(k_gather, dim3(nb), dim3(NT), 0, s, h->g0, h->gh, d_rhs, (const unsigned char *)h->part, h->b,
-                       (double *)nullptr);
+                       (double *)nullptr, (double *)nullptr);
     hipLaunchKernelGGL(k_gather, dim3(nb), dim3(NT), 0, s, h->g0, h->gh, d_sol, (const unsigned char *)h->part, h->x,
-                       (double *)nullptr);
+                       (double *)nullptr, (double *)nullptr);
     exact_residual(h, d_res, S_RRT);
     HIPCHK(hipGetLastError());
     int rc = read_scal(h);
