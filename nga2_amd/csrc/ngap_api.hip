@@ -1152,7 +1152,17 @@ void launch_bottom_levels(ngap_t *h, int lb) {
     launch_bottom<T>(h->stream, a);
 }
 
-constexpr long long PAIR_MIN_CELLS = 1LL << 24;  // levels whose post-smoothing pairs are fused
+// Levels whose sweeps run in fused pairs. With k_sweep2_pair (pair_form) from
+// 2^19 cells on: 256^3 channel, FP32 V(2,2), 22.17 ms a solve with pairs on the
+// fine level only, 21.05 from 2^23, 20.21 from 2^20, 20.10 from 2^19 and 2^18,
+// 20.25 from 2^16 (implicit 128^3: 5.17, 5.24, 4.90, 4.78, 4.84, 4.88 ms); below,
+// a launch has too few planes per chunk and too few workgroups. With k_sweep2 on
+// the largest levels only: at 256^3 the pair took 244 us against 2 x 131, and it
+// was slower on the smaller ones.
+template <typename T>
+static bool pairs_on(const Geo &g) {
+    return g.N >= (pair_form<T>(g) ? 1LL << 19 : 1LL << 24);
+}
 // Levels whose first pre-smoothing sweep (from a zero iterate) runs as the
 // whole-row sweep kernel rather than the stencil form: rows of <= 128 cells,
 // >= 2^20 cells. The stencil reads f and c at every neighbour to form f / c;
@@ -1170,16 +1180,14 @@ void vcycle(ngap_t *h, const T *f0, T *v0) {
     const int nl = h->nlev;
     hipStream_t s = h->stream;
     const int npre = h->opts.nu_pre, npost = h->opts.nu_post;
-    // On levels of >= PAIR_MIN_CELLS cells the post-smoothing sweeps run in
-    // fused pairs (one launch each) plus a single one for an odd count; every
-    // launch switches the level's buffer. At 256^3 the pair takes 244 us
-    // against 2 x 131 us on the fine level, but is slower on the smaller
-    // levels, whose chunks are too short to amortise its deeper pipeline.
-    auto post_launches = [&](const Level &L) { return L.g.N >= PAIR_MIN_CELLS ? npost / 2 + (npost & 1) : npost; };
+    // On the levels of pairs_on the post-smoothing sweeps run in fused pairs
+    // (one launch each) plus a single one for an odd count; every launch
+    // switches the level's buffer.
+    auto post_launches = [&](const Level &L) { return pairs_on<T>(L.g) ? npost / 2 + (npost & 1) : npost; };
     // pre-smoothing on those levels: the first two sweeps (from a zero
     // iterate) as one pair launch, the rest as in the post-smoothing
     auto pre_launches = [&](const Level &L) {
-        if (L.g.N < PAIR_MIN_CELLS || npre < 2) return npre;
+        if (!pairs_on<T>(L.g) || npre < 2) return npre;
         return 1 + (npre - 2) / 2 + ((npre - 2) & 1);
     };
     const int lb = bottom_start<T>(h);
@@ -1199,7 +1207,7 @@ void vcycle(ngap_t *h, const T *f0, T *v0) {
             continue;
         }
         const int npl = post_launches(L), prl = pre_launches(L);
-        const bool pairs = L.g.N >= PAIR_MIN_CELLS;
+        const bool pairs = pairs_on<T>(L.g);
         T *bufs[2] = {((prl + npl) & 1) ? fin : D.w, ((prl + npl) & 1) ? D.w : fin};
         const T *cur = nullptr;
         int nb = 0;
@@ -1252,7 +1260,7 @@ void vcycle(ngap_t *h, const T *f0, T *v0) {
         launch_prolong_to<T>(s, L.g, Cn.g, L.cdir, DC.pm, DC.pp, DC.v, cur, cur);
         for (int sw = 0; sw < npost;) {
             T *nxt = (cur == fin) ? D.w : fin;
-            if (npost - sw >= 2 && L.g.N >= PAIR_MIN_CELLS) {
+            if (npost - sw >= 2 && pairs_on<T>(L.g)) {
                 launch_sweep2<T>(s, L.g, D.c, D.a0, D.a1, D.a2, f, cur, nxt, 1);
                 sw += 2;
             } else {
@@ -2375,12 +2383,13 @@ static int t_rbgs(ngap_t *h, int l, const double *f, double *v, int order) {
     if (!rc) rc = up<T>(h->stream, tmp, v, n, &dv);
     if (rc || !dout) return rc ? rc : NGAP_ERR_ALLOC;
     if ((order & 6) == 6)  // the first two sweeps from a zero iterate in one launch
-        launch_sweep2<T>(h->stream, L.g, D.c, D.a0, D.a1, D.a2, df, (const T *)nullptr, dout, order & 1);
+        launch_sweep2<T>(h->stream, L.g, D.c, D.a0, D.a1, D.a2, df, (const T *)nullptr, dout, order & 1,
+                         (order & 8) != 0);
     else if (order & 2)  // first sweep from a zero iterate (the V-cycle's pre-smoothing)
         launch_smooth0<T>(h->stream, L.g, D.c, D.a0, D.a1, D.a2, df, dout, order & 1);
     else if (order & 4)  // two sweeps of the same order in one launch (the post-smoothing pair)
-        launch_sweep2<T>(h->stream, L.g, D.c, D.a0, D.a1, D.a2, df, dv, dout, order & 1);
-    else  // bit 3: the 64-wide tiles on every level; bit 4: the single sweep from a zero iterate
+        launch_sweep2<T>(h->stream, L.g, D.c, D.a0, D.a1, D.a2, df, dv, dout, order & 1, (order & 8) != 0);
+    else  // bit 3: the 64-wide tiles (pairs: one cell per lane) on every level; bit 4: the single sweep from a zero iterate
         launch_sweep<T>(h->stream, L.g, D.c, D.a0, D.a1, D.a2, df, (order & 16) ? (const T *)nullptr : dv, dout,
                         order & 1, (order & 8) != 0);
     HIPCHK(hipGetLastError());

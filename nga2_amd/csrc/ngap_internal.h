@@ -24,11 +24,20 @@ void launch_apply_x32(hipStream_t s, const Geo &g, const double *c, const double
 // <= 128 cells run whole-row tiles (k_sweep_row) unless tiles is set.
 template <typename T>
 void launch_sweep(hipStream_t s, const Geo &g, const T *c, const T *a0, const T *a1, const T *a2, const T *f,
-                  const T *vin, T *vout, int c1, bool tiles = false);
-// two fused sweeps of the same colour order (vin != vout)
+                  const T *vin, T *vout, int c1, bool one_cell = false);
+// true where launch_sweep2 can take k_sweep2_pair: FP32, even row length, and
+// even counts where periodic (an odd one has no red-black order across the wrap;
+// k_sweep2 colours by the wrapped index). Offsets in a plane are 32 bits of bytes.
+template <typename T>
+inline bool pair_form(const Geo &g) {
+    return sizeof(T) == 4 && g.n0 % 2 == 0 && !(g.p1 && (g.n1 & 1)) && !(g.p2 && (g.n2 & 1)) &&
+           (long long)g.n0 * g.n1 < (1LL << 30);
+}
+// two fused sweeps of the same colour order (vin != vout); one_cell: the
+// one-cell-per-lane kernel on every level
 template <typename T>
 void launch_sweep2(hipStream_t s, const Geo &g, const T *c, const T *a0, const T *a1, const T *a2, const T *f,
-                   const T *vin, T *vout, int c1);
+                   const T *vin, T *vout, int c1, bool one_cell = false);
 // first symmetric sweep from a zero iterate as a stencil (no LDS)
 template <typename T>
 void launch_smooth0(hipStream_t s, const Geo &g, const T *c, const T *a0, const T *a1, const T *a2, const T *f, T *v,

@@ -961,6 +961,237 @@ __global__ void __launch_bounds__(SX *SY) k_sweep2(Geo g, const T *__restrict__ 
     }
 }
 
+// ------------------------------------------------------------------ the pair, two cells per lane
+// The pair of k_sweep2 in FP32 on levels of an even row length. In k_sweep2 a
+// lane holds one cell column and half of the lanes idle: at the step whose
+// newest plane is P, h1 on P, h2 on P-1, h3 on P-2 and h4 on P-3 all fall on
+// the columns of one x-y parity, and on the others' at the next step. Its
+// vector instructions alone took 156 of the 247 us of a 256^3 launch. Here a
+// lane holds both columns of an x pair, A and B; at every step one of them (X)
+// does all four half-steps and the other (Y) none, so no lane idles.
+// - In-plane x neighbours: the other column's values of the previous step, its
+//   own (a register) and the adjacent lane's (a lane shift; no LDS).
+// - y neighbours and a_y through LDS, one value per pair and field (the field
+//   exists on one colour only): 80 KB.
+// - A tile is 64 x 32 cells: 16 waves, wave w holding rows w and w + 16 (equal
+//   parity, so that which of the pair is A is the same for the whole wave and a
+//   template argument, S = its x parity). The ring is 4 cells wide, so the
+//   outermost cells only hand on vin and nothing outside the tile is read:
+//   output core 56 x 24.
+// - No cell is masked: outside a wall f, a are 0 and c is 1, which gives 0, and
+//   what the tile's outermost cells compute from neighbours they do not have
+//   stays inside the ring.
+// - Loads are issued two planes ahead, each of an x pair (8 bytes) and all of
+//   them unconditional: buffer loads, whose offsets past the plane give 0 (and
+//   whose stores there are dropped). Behind branches the wait for the planes of
+//   the last step became a wait for those just issued (215 us).
+// - Six steps per loop iteration: the life of a loaded value, so that the queues
+//   shift by renaming (a copy of a load in flight waits for it), and of the
+//   LDS slots, so that their addresses are constants.
+// Of the 142 us, the loads with their halos take about 110 at 5.5 TB/s, the
+// vector instructions about 60. Per cell the operations and roundings of k_sweep2, so bit-identical to it.
+// 256^3: 247 -> 145 us, from zero 209 -> 142 us.
+constexpr int PX = 64, PY = 32, PR = 4;
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ float lane_down(float v) {  // from lane - 1
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float lane_up(float v) {  // from lane + 1
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x130, 0xf, 0xf, true));
+}
+
+struct PairLds {
+    float a1[6][2][PY][PX / 2];  // a_y of six planes, even and odd cells
+    float h[3][2][PY][PX / 2];   // fields h1, h2, h3, two planes
+    float v[2][PY][PX / 2];      // vin of two planes (the second colour's cells)
+};
+
+template <bool ZERO_IN, int S>
+__device__ __forceinline__ void pair_march(PairLds &M, const Geo &g, const float *__restrict__ c,
+                                           const float *__restrict__ a0, const float *__restrict__ a1,
+                                           const float *__restrict__ a2, const float *__restrict__ f,
+                                           const float *__restrict__ vin, float *__restrict__ vout, int k0, int k1,
+                                           int ty, int q, bool valid, unsigned oE, unsigned oS) {
+#pragma clang fp contract(off)
+    const int n2 = g.n2, per2 = g.p2;
+    const long long plane = (long long)g.n0 * g.n1;
+    const unsigned bytes = 4u * (unsigned)plane;
+    // the pair at element offset o (a plane's first); zero outside the plane's
+    // bytes and for n == 0
+    auto at2 = [&](const float *p, long long o, unsigned n) -> f32x2 {
+        __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)(p + o), 0, (int)n, 0x00027000);
+        return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(r, (int)oE, 0, 0));
+    };
+    // c, f, a0 of planes P+2 .. P-3, a1 of P+2 .. P, a2 of P+2 .. P-3 and P+3's at
+    // the end of a step, of both columns; vin of the second colour's, P+3 .. P-1
+    f32x2 cq[6], fq[6], a0q[6], a1q[3], a2q[7];
+    float w[5];
+#pragma unroll
+    for (int i = 0; i < 6; i++) {
+        cq[i] = f32x2{1.0f, 1.0f};
+        fq[i] = a0q[i] = f32x2{0.0f, 0.0f};
+    }
+#pragma unroll
+    for (int i = 0; i < 7; i++) a2q[i] = f32x2{0.0f, 0.0f};
+    a1q[2] = f32x2{0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < 5; i++) w[i] = 0.0f;
+    float h1[2] = {0.0f, 0.0f}, h2[2] = {0.0f, 0.0f}, h3[2] = {0.0f, 0.0f};  // of the last two steps
+    int P = k0 - 3;
+    // before the first step, queues as the step's shift expects them: planes P+1,
+    // P of c, f, a0, a1 and P+2 .. P of a2, P+2 .. P-1 of vin. The column active
+    // at plane P is A, so the second colour's is B there and at P+2.
+#pragma unroll
+    for (int i = 3; i >= 0; i--) {
+        const int kk = wrapc(P + 2 - i, n2, per2);
+        const long long o = kk < 0 ? 0 : kk * plane;
+        const unsigned n = kk < 0 ? 0 : bytes;
+        if (i == 1 || i == 2) {
+            cq[i - 1] = at2(c, o, n);
+            fq[i - 1] = at2(f, o, n);
+            a0q[i - 1] = at2(a0, o, n);
+            a1q[i - 1] = at2(a1, o, n);
+        }
+        if (i < 3) a2q[i] = at2(a2, o, n);
+        if (!ZERO_IN) w[i] = at2(vin, o, n)[(i & 1) ? S : 1 - S];
+    }
+    // planes P + 2 and P + 3: element offset and bytes (0 outside a wall)
+    int kM = per2 ? wrapc(P + 3, n2, 1) : P + 3;
+    const int kN = wrapc(P + 2, n2, per2);
+    long long oN = kN * plane, oM = kM * plane;
+    unsigned nN = kN < 0 ? 0 : bytes;
+    const unsigned out = valid ? 0u : 0x40000000u;
+    // one step; m: its number modulo 6, even where column A is active
+    auto step = [&](auto mc) {
+        constexpr int m = decltype(mc)::value, X = m & 1, Y = 1 - X, x = X ^ S, y = 1 - x;  // x: the active cell's parity
+        const bool ok = (unsigned)(per2 ? 0 : P) + out < (unsigned)n2;
+#pragma unroll
+        for (int i = 5; i > 0; i--) {
+            cq[i] = cq[i - 1];
+            fq[i] = fq[i - 1];
+            a0q[i] = a0q[i - 1];
+        }
+#pragma unroll
+        for (int i = 6; i > 0; i--) a2q[i] = a2q[i - 1];
+#pragma unroll
+        for (int i = 4; i > 0; i--) w[i] = w[i - 1];
+        a1q[2] = a1q[1];
+        a1q[1] = a1q[0];
+        cq[2][0] = ok ? cq[2][0] : 1.0f;
+        cq[2][1] = ok ? cq[2][1] : 1.0f;
+        // publish plane P
+        M.a1[m][0][ty][q] = a1q[2][0];
+        M.a1[m][1][ty][q] = a1q[2][1];
+        if (!ZERO_IN) M.v[m & 1][ty][q] = w[3];
+        __builtin_amdgcn_sched_barrier(0);
+        // plane P+2, and vin of P+3 (its second colour's column is X)
+        const long long oL = oM;
+        const unsigned nL = (unsigned)kM < (unsigned)n2 ? bytes : 0;
+        cq[0] = at2(c, oN, nN);
+        fq[0] = at2(f, oN, nN);
+        a0q[0] = at2(a0, oN, nN);
+        a1q[0] = at2(a1, oN, nN);
+        if (!ZERO_IN) w[0] = at2(vin, oL, nL)[x];
+        __builtin_amdgcn_sched_barrier(0);
+        lds_barrier();
+        constexpr int m1 = (m + 5) % 6, m2 = (m + 4) % 6, m3 = (m + 3) % 6;
+        const int tm = ty > 0 ? ty - 1 : 0, tp = ty < PY - 1 ? ty + 1 : PY - 1;
+        // one half-step of column X at plane P - d: y neighbours from F, own: the
+        // other column's value there, z neighbours zm / zp
+        auto half = [&](auto dd, int sl, const float (*F)[PX / 2], float own, float zm, float zp) -> float {
+            constexpr int d = decltype(dd)::value;
+            const float ym = F[tm][q], yp = F[tp][q], b1 = M.a1[sl][x][ty][q], b1p = M.a1[sl][x][tp][q];
+            const float a0y = a0q[2 + d][y];
+            const float xm = x == 0 ? lane_down(own) : own, xp = x == 0 ? own : lane_up(own);
+            const float a0p = x == 0 ? a0y : lane_up(a0y);
+            float sum = fq[2 + d][x];
+            sum = fma_t(-a0q[2 + d][x], xm, sum);
+            sum = fma_t(-a0p, xp, sum);
+            sum = fma_t(-b1, ym, sum);
+            sum = fma_t(-b1p, yp, sum);
+            sum = fma_t(-a2q[3 + d][x], zm, sum);
+            sum = fma_t(-a2q[2 + d][x], zp, sum);
+            return sum / cq[2 + d][x];
+        };
+        using I0 = std::integral_constant<int, 0>;
+        using I1 = std::integral_constant<int, 1>;
+        using I2 = std::integral_constant<int, 2>;
+        using I3 = std::integral_constant<int, 3>;
+        const float u1 = ZERO_IN ? fq[2][x] / cq[2][x] : half(I0(), m, M.v[m & 1], w[3], w[4], w[2]);
+        const float u2 = half(I1(), m1, M.h[0][m1 & 1], h1[0], h1[1], u1);
+        const float u3 = half(I2(), m2, M.h[1][m1 & 1], h2[0], h2[1], u2);
+        const float u4 = half(I3(), m3, M.h[2][m1 & 1], h3[0], h3[1], u3);
+        // read at the next step, after its barrier
+        M.h[0][m & 1][ty][q] = u1;
+        M.h[1][m & 1][ty][q] = u2;
+        M.h[2][m & 1][ty][q] = u3;
+        // plane P - 3: h4 on X, h3 (of the last step) on Y; dropped outside the core
+        // and the chunk's planes
+        {
+            f32x2 o;
+            o[0] = x == 0 ? u4 : h3[0];
+            o[1] = x == 0 ? h3[0] : u4;
+            const int s = P - 3;
+            const bool sin = s >= k0 && s < k1;
+            __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)(vout + (sin ? s : 0) * plane), 0,
+                                                                         sin ? (int)bytes : 0, 0x00027000);
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, o), r, (int)oS, 0, 0);
+        }
+        h1[1] = h1[0];
+        h1[0] = u1;
+        h2[1] = h2[0];
+        h2[0] = u2;
+        h3[1] = h3[0];
+        h3[0] = u3;
+        // a2 of P+3 after the last use of P-3's, so that its registers are free
+        __builtin_amdgcn_sched_barrier(0);
+        a2q[0] = at2(a2, oL, nL);
+        __builtin_amdgcn_sched_barrier(0);
+        oN = oL;
+        nN = nL;
+        const bool wrap = per2 && kM + 1 == n2;
+        kM = wrap ? 0 : kM + 1;
+        oM = wrap ? 0 : oM + plane;
+        P++;
+    };
+    // six steps: the period of the queues' registers and of the LDS slots
+    while (P - 3 < k1) {
+        step(std::integral_constant<int, 0>());
+        step(std::integral_constant<int, 1>());
+        step(std::integral_constant<int, 2>());
+        step(std::integral_constant<int, 3>());
+        step(std::integral_constant<int, 4>());
+        step(std::integral_constant<int, 5>());
+    }
+}
+
+template <bool ZERO_IN>
+__global__ void __launch_bounds__(1024) k_sweep2_pair(Geo g, const float *__restrict__ c, const float *__restrict__ a0,
+                                                      const float *__restrict__ a1, const float *__restrict__ a2,
+                                                      const float *__restrict__ f, const float *__restrict__ vin,
+                                                      float *__restrict__ vout, int c1, int kc, int gx, int gy) {
+    __shared__ PairLds M;
+    int bx, by, bz;
+    tile_of(gx, gy, bx, by, bz);
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int q = lane & 31, ty = wv + 16 * (lane >> 5);
+    const int iu = bx * (PX - 2 * PR) - PR + 2 * q, ju = by * (PY - 2 * PR) - PR + ty;
+    const int ii = wrapc(iu, g.n0, g.p0), jj = wrapc(ju, g.n1, g.p1);
+    const bool valid = ii >= 0 && jj >= 0;
+    const unsigned oE = valid ? 4u * (unsigned)(jj * g.n0 + ii) : 0xFFFFFFF8u;
+    const bool core = 2 * q >= PR && 2 * q < PX - PR && ty >= PR && ty < PY - PR && iu < g.n0 && ju < g.n1;
+    const unsigned oS = core ? oE : 0xFFFFFFF8u;
+    const int k0 = bz * kc, k1 = min(g.n2, k0 + kc);
+    // colour (x + j + k) & 1 of the cell that is A at the first plane, k0 - 3
+    const int S = (c1 + by * (PY - 2 * PR) - PR + wv + k0 - 3) & 1;
+    if (S == 0)
+        pair_march<ZERO_IN, 0>(M, g, c, a0, a1, a2, f, vin, vout, k0, k1, ty, q, valid, oE, oS);
+    else
+        pair_march<ZERO_IN, 1>(M, g, c, a0, a1, a2, f, vin, vout, k0, k1, ty, q, valid, oE, oS);
+}
+
 // ------------------------------------------------------------------ restriction
 __device__ __forceinline__ int gdim_(const Geo &g, int d) { return d == 0 ? g.n0 : (d == 1 ? g.n1 : g.n2); }
 __device__ __forceinline__ int gper_(const Geo &g, int d) { return d == 0 ? g.p0 : (d == 1 ? g.p1 : g.p2); }
@@ -1722,13 +1953,36 @@ void launch_sweep(hipStream_t s, const Geo &g, const T *c, const T *a0, const T 
         launch_sweep_sy<T, 16>(s, g, c, a0, a1, a2, f, vin, vout, c1, 512);
 }
 
-// Two sweeps of colour order c1 in one launch (k_sweep2): 58 x 10 output
+// Two sweeps of colour order c1 in one launch: k_sweep2_pair where it can run
+// (247 -> 145 us at 256^3), else k_sweep2, 58 x 10 output
 // tiles, about 512 workgroups, z chunks of >= 16 planes on large levels (each
 // chunk recomputes 6 planes). vin and vout must differ; vin == nullptr: the
 // first sweep starts from a zero iterate.
 template <typename T>
 void launch_sweep2(hipStream_t s, const Geo &g, const T *c, const T *a0, const T *a1, const T *a2, const T *f,
-                   const T *vin, T *vout, int c1) {
+                   const T *vin, T *vout, int c1, bool one_cell) {
+    if constexpr (std::is_same<T, float>::value) {
+        // (8-byte accesses; the level's own buffers always are aligned)
+        const auto al = reinterpret_cast<uintptr_t>(c) | reinterpret_cast<uintptr_t>(a0) |
+                        reinterpret_cast<uintptr_t>(a1) | reinterpret_cast<uintptr_t>(a2) |
+                        reinterpret_cast<uintptr_t>(f) | reinterpret_cast<uintptr_t>(vin) |
+                        reinterpret_cast<uintptr_t>(vout);
+        if (!one_cell && pair_form<T>(g) && al % 8 == 0) {
+            const int gx = (g.n0 + PX - 2 * PR - 1) / (PX - 2 * PR), gy = (g.n1 + PY - 2 * PR - 1) / (PY - 2 * PR);
+            // one workgroup per CU: z chunks so that about 256 run, each of whole
+            // rounds of 6 steps and recomputing 6 planes
+            const long long gz = std::max<long long>(1, 256 / ((long long)gx * gy));
+            const int kc = (int)(((g.n2 + gz - 1) / gz + 5) / 6 * 6);
+            const int nz = (g.n2 + kc - 1) / kc;
+            if (vin)
+                hipLaunchKernelGGL(k_sweep2_pair<false>, dim3((unsigned)(gx * gy * nz)), dim3(1024), 0, s, g, c, a0, a1,
+                                   a2, f, vin, vout, c1, kc, gx, gy);
+            else
+                hipLaunchKernelGGL(k_sweep2_pair<true>, dim3((unsigned)(gx * gy * nz)), dim3(1024), 0, s, g, c, a0, a1,
+                                   a2, f, vin, vout, c1, kc, gx, gy);
+            return;
+        }
+    }
     constexpr int SY = 16;
     const int gx = (g.n0 + SX - 2 * R2 - 1) / (SX - 2 * R2), gy = (g.n1 + SY - 2 * R2 - 1) / (SY - 2 * R2);
     const long long tiles = (long long)gx * gy;
@@ -1795,7 +2049,7 @@ template void launch_bottom<float>(hipStream_t, const BotArgs<float> &);
     template void launch_sweep<T>(hipStream_t, const Geo &, const T *, const T *, const T *, const T *, const T *, \
                                   const T *, T *, int, bool);                                                      \
     template void launch_sweep2<T>(hipStream_t, const Geo &, const T *, const T *, const T *, const T *,          \
-                                   const T *, const T *, T *, int);                                                \
+                                   const T *, const T *, T *, int, bool);                                          \
     template void launch_smooth0<T>(hipStream_t, const Geo &, const T *, const T *, const T *, const T *,          \
                                     const T *, T *, int);                                                          \
     template void launch_resid<T>(hipStream_t, const Geo &, const T *, const T *, const T *, const T *, const T *, \
