@@ -1,26 +1,35 @@
 // fourier3d on the GPU: the FFT direct solve of a circulant stencil operator
-// on a periodic uniform grid (fourier3d_class.f90:1103-1202), with rocFFT
-// (through hipFFT) for the transforms and HIP kernels for everything around
-// them: the circulance check, the placement of the stencil, the inversion of
-// the transformed operator, the spectral divide, the copy of the solution into
-// sol and its ghost fill.
+// on a periodic uniform grid (fourier3d_class.f90:1103-1202): the circulance
+// check, the placement of the stencil, the inversion of the transformed
+// operator, the transforms with the spectral divide, the copy of the solution
+// into sol and its ghost fill.
 //
 // The transforms are real-to-complex over the directions with more than one
-// cell, slowest first (z, y, x). The forward one reads the interior of the
-// caller's ghosted rhs in place (strided plan layout); the inverse one writes
-// a dense array (rocFFT's two-dimensional complex-to-real plans with a
-// strided output fail to execute), which one pass copies into the interior
-// of sol. A solve is: forward transform, one pass over the half spectrum
-// (zero mode, 1/F, normalisation), inverse transform, copy, ghost fill.
+// cell, x first. Where x is one of them and every length is a product of 2, 3,
+// 5, 7, 11 and 13 of at most FFT_MAX, they are the kernels of this file: a
+// solve is five passes over memory (x forward, y forward, z forward with the
+// divide and z inverse, y inverse, x inverse into sol and its ghosts). 256^3:
+// 346 us a solve, with the library 581; 90 x 75 x 64: 60 and 77 us. Against a
+// solve in extended precision their error is about half of the library's
+// (geometric mean over 90 grids of one to three directions).
+//
+// Elsewhere rocFFT (through hipFFT) transforms. The forward plan reads the
+// interior of the caller's ghosted rhs in place (strided plan layout); the
+// inverse one writes a dense array (rocFFT's two-dimensional complex-to-real
+// plans with a strided output fail to execute), which one pass copies into the
+// interior of sol. A solve is: forward transform, one pass over the half
+// spectrum (zero mode, 1/F, normalisation), inverse transform, copy, ghost fill.
 // The half spectrum (last transformed direction n/2+1 long) holds every mode
 // of the reference's full complex transform, since F(-k) = conj F(k) for a
 // real stencil and a real right-hand side.
 #include <hip/hip_runtime.h>
 #include <hipfft/hipfft.h>
 
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
 #include <cstdio>
+#include <type_traits>
 #include <vector>
 
 #include "ngapfft.h"
@@ -97,11 +106,13 @@ __global__ void k_place(Grid g, int nst, const int *__restrict__ stc, const doub
 
 // zero mode to 1, count |F| < 1000 eps, invert, count NaN
 // (fourier3d_class.f90:1142-1160)
-__global__ void __launch_bounds__(PT) k_invert(long long M, double2 *__restrict__ F, int *__restrict__ part_small,
-                                               int *__restrict__ part_nan) {
+// (rows of `pitch` modes, `len` of them in use)
+__global__ void __launch_bounds__(PT) k_invert(long long M, int pitch, int len, double2 *__restrict__ F,
+                                               int *__restrict__ part_small, int *__restrict__ part_nan) {
     __shared__ int s0[PT], s1[PT];
     int small = 0, nan = 0;
     for (long long m = blockIdx.x * (long long)PT + threadIdx.x; m < M; m += (long long)gridDim.x * PT) {
+        if (m % pitch >= len) continue;
         double2 f = F[m];
         if (m == 0) f = make_double2(1.0, 0.0);
         if (hypot(f.x, f.y) < 1000.0 * DBL_EPSILON) small++;
@@ -180,6 +191,360 @@ __global__ void __launch_bounds__(PT) k_sync_dir(Grid g, int ax, double *a) {
     }
 }
 
+// ------------------------------------------------------------------ transforms in LDS
+// A transform of length n = r_0 r_1 ... (r of 2, 3, 4, 5, 7, 8, 11, 13; n <=
+// FFT_MAX) decimated in frequency: pass p combines the r_p elements m_p =
+// n / (r_0 .. r_p) apart and stores them where they were, so that a tile of
+// lines is transformed in place in LDS with one barrier a pass; the first pass
+// reads from memory and the last one writes to it. The modes end up in
+// digit-reversed order and stay there: the operator's transform has the same
+// order, the divide is pointwise, and the inverse runs the passes backwards.
+constexpr int FFT_MAX = 1024;  // 8 lines of 16 bytes a cell: 128 KB of LDS
+constexpr int FT = 256;                // threads of a workgroup at most
+constexpr int LB = 3, LINES = 1 << LB;  // lines of a column tile
+struct FftDim {
+    int n, np;
+    int r[10], m[10];
+    unsigned magic[10];  // 2^32 / m rounded up: g / m for g m < 2^32, m > 1
+    const double2 *w;    // exp(-2 pi i k / n), k < n
+    const unsigned short *pos;  // where mode k is
+};
+
+__device__ __forceinline__ double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
+__device__ __forceinline__ double2 csub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
+__device__ __forceinline__ double2 cmul(double2 a, double2 b) {
+    return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+}
+__device__ __forceinline__ double2 cmulc(double2 a, double2 b) {  // a conj(b)
+    return make_double2(a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y);
+}
+template <bool INV>
+__device__ __forceinline__ double2 mul_i(double2 a) {  // by -i (forward), i (inverse)
+    return INV ? make_double2(-a.y, a.x) : make_double2(a.y, -a.x);
+}
+
+template <bool INV>
+__device__ __forceinline__ void dft4(double2 &a, double2 &b, double2 &c, double2 &d) {
+    const double2 s0 = cadd(a, c), d0 = csub(a, c), s1 = cadd(b, d), d1 = mul_i<INV>(csub(b, d));
+    a = cadd(s0, s1);
+    c = csub(s0, s1);
+    b = cadd(d0, d1);
+    d = csub(d0, d1);
+}
+
+// v_k = sum_q v_q w^(qk), w the R-th root of unity; w: the table of n, whose
+// entries n/R apart are that root's powers
+template <int R, bool INV>
+__device__ __forceinline__ void dft(double2 (&v)[R], const double2 *w, int n) {
+    if constexpr (R == 2) {
+        const double2 t = csub(v[0], v[1]);
+        v[0] = cadd(v[0], v[1]);
+        v[1] = t;
+    } else if constexpr (R == 4) {
+        dft4<INV>(v[0], v[1], v[2], v[3]);
+    } else if constexpr (R == 8) {
+        constexpr double h = 0.70710678118654752440;  // sqrt(1/2)
+        dft4<INV>(v[0], v[2], v[4], v[6]);
+        dft4<INV>(v[1], v[3], v[5], v[7]);
+        const double2 t = mul_i<INV>(v[3]), u = mul_i<INV>(v[7]);
+        const double2 o1 = make_double2(h * (v[3].x + t.x), h * (v[3].y + t.y));
+        const double2 o2 = mul_i<INV>(v[5]);
+        const double2 o3 = make_double2(h * (u.x - v[7].x), h * (u.y - v[7].y));
+        const double2 e0 = v[0], e1 = v[2], e2 = v[4], e3 = v[6], o0 = v[1];
+        v[0] = cadd(e0, o0);
+        v[4] = csub(e0, o0);
+        v[1] = cadd(e1, o1);
+        v[5] = csub(e1, o1);
+        v[2] = cadd(e2, o2);
+        v[6] = csub(e2, o2);
+        v[3] = cadd(e3, o3);
+        v[7] = csub(e3, o3);
+    } else {
+        // odd: sums and differences of the pairs q, R - q against cosines and sines
+        constexpr int H = (R - 1) / 2;
+        double2 s[H], d[H], c[H];
+        const int step = n / R;
+#pragma unroll
+        for (int q = 0; q < H; q++) {
+            s[q] = cadd(v[q + 1], v[R - 1 - q]);
+            d[q] = csub(v[q + 1], v[R - 1 - q]);
+            c[q] = w[(q + 1) * step];
+        }
+        double2 t = v[0];
+#pragma unroll
+        for (int q = 0; q < H; q++) t = cadd(t, s[q]);
+        const double2 x0 = v[0];
+        v[0] = t;
+#pragma unroll
+        for (int k = 1; k <= H; k++) {
+            double2 e = x0, o = make_double2(0.0, 0.0);
+#pragma unroll
+            for (int q = 1; q <= H; q++) {
+                const int x = q * k % R, z = x <= H ? x : R - x;  // a folded constant
+                const double cs = c[z - 1].x, sn = x <= H ? c[z - 1].y : -c[z - 1].y;
+                e.x += s[q - 1].x * cs;
+                e.y += s[q - 1].y * cs;
+                o.x += d[q - 1].x * sn;
+                o.y += d[q - 1].y * sn;
+            }
+            // i o (forward; the table's sines are already negative), -i o (inverse)
+            const double2 io = INV ? make_double2(o.y, -o.x) : make_double2(-o.y, o.x);
+            v[k] = cadd(e, io);
+            v[R - k] = csub(e, io);
+        }
+    }
+}
+
+// one butterfly's r elements: twiddles before the inverse, after the forward one
+template <int R, bool INV>
+__device__ __forceinline__ void butterfly(double2 (&v)[R], const double2 *w, int n, int j, int m) {
+    const int lj = n / (R * m) * j;
+    if (INV) {
+#pragma unroll
+        for (int q = 1; q < R; q++) v[q] = cmulc(v[q], w[lj * q]);
+        dft<R, true>(v, w, n);
+    } else {
+        dft<R, false>(v, w, n);
+#pragma unroll
+        for (int q = 1; q < R; q++) v[q] = cmul(v[q], w[lj * q]);
+    }
+}
+
+__device__ __forceinline__ int div_m(int g, int m, unsigned magic) { return m == 1 ? g : (int)__umulhi((unsigned)g, magic); }
+
+// BIG: with the radices 7, 11 and 13, which take up to twice the registers
+template <bool BIG, typename Run>
+__device__ __forceinline__ void by_radix(int r, Run run) {
+    if (r == 8) {
+        run(std::integral_constant<int, 8>());
+    } else if (r == 4) {
+        run(std::integral_constant<int, 4>());
+    } else if (r == 2) {
+        run(std::integral_constant<int, 2>());
+    } else if (r == 3) {
+        run(std::integral_constant<int, 3>());
+    } else if (!BIG || r == 5) {
+        run(std::integral_constant<int, 5>());
+    } else if constexpr (BIG) {
+        if (r == 7)
+            run(std::integral_constant<int, 7>());
+        else if (r == 11)
+            run(std::integral_constant<int, 11>());
+        else
+            run(std::integral_constant<int, 13>());
+    }
+}
+
+// Lines across rows (y and z). A workgroup transforms 8 adjacent ones:
+// whole 128-byte lines of every row, a row of the half spectrum being padded to
+// 8 modes for that. FWD and INV in place; DIVIDE: forward, times finv, inverse,
+// in one pass over memory, the last forward and the first inverse pass in
+// registers. line l of outer o starts at o * ostride + l; its elements are es
+// apart; lines whose x is padding are left out.
+// Bound by memory: at 256^3 (129 x 256 x 256 modes, 270 MB in and out) 55 us a plain
+// pass, the library's 82; the divide (405 MB) 103 us, two library passes and a
+// divide 221.
+enum { FWD, INV, DIVIDE };
+template <int MODE, bool BIG>
+__global__ void __launch_bounds__(FT, BIG ? 2 : 4) k_fft_col(FftDim D, const double2 *__restrict__ finv, double2 *a, int nlines,
+                                                long long es, long long ostride, int pitch, int nxh,
+                                                double scale) {
+    extern __shared__ double2 sm[];
+    const int n = D.n, T = blockDim.x;
+    double2 *w = sm, *t = sm + n;
+    for (int i = threadIdx.x; i < n; i += T) w[i] = D.w[i];
+    const int c = threadIdx.x & (LINES - 1), g0 = threadIdx.x >> LB, gs = T >> LB;
+    const int line = blockIdx.x * LINES + c;
+    const bool on = line < nlines && line % pitch < nxh;
+    const long long base = (long long)blockIdx.y * ostride + line;
+    const bool zero = base == 0;  // the line of the zero mode
+    double2 *__restrict__ p = a + base;
+    const double2 *__restrict__ fi = MODE == DIVIDE ? finv + base : nullptr;
+    __syncthreads();
+    const int np = D.np;
+    const int total = MODE == DIVIDE ? 2 * np - 1 : np;
+    for (int k = 0; k < total; k++) {
+        // the pass of this step and where its elements are
+        const bool inv = MODE == INV || (MODE == DIVIDE && k >= np);
+        const int ps = MODE == INV ? np - 1 - k : (MODE == DIVIDE && k >= np ? 2 * np - 2 - k : k);
+        const bool in = k == 0, out = k == total - 1, mid = MODE == DIVIDE && k == np - 1;
+        const int r = D.r[ps], m = D.m[ps];
+        const unsigned magic = D.magic[ps];
+        const int ng = n / r;
+        auto run = [&](auto rc) {
+            constexpr int R = decltype(rc)::value;
+            if (!on) return;
+            for (int g = g0; g < ng; g += gs) {
+                const int l = div_m(g, m, magic), j = g - l * m, b = l * R * m + j;
+                double2 v[R];
+#pragma unroll
+                for (int q = 0; q < R; q++) v[q] = in ? p[(b + q * m) * es] : t[((b + q * m) << LB) + c];
+                if (mid) {
+                    double2 f[R];
+#pragma unroll
+                    for (int q = 0; q < R; q++) f[q] = fi[(b + q * m) * es];
+                    dft<R, false>(v, w, n);  // the last pass: m = 1, no twiddles
+#pragma unroll
+                    for (int q = 0; q < R; q++) {
+                        v[q] = cmul(v[q], f[q]);
+                        v[q].x *= scale;
+                        v[q].y *= scale;
+                    }
+                    if (zero && b == 0) v[0] = make_double2(0.0, 0.0);
+                    dft<R, true>(v, w, n);
+                } else if (MODE != FWD && inv) {
+                    butterfly<R, true>(v, w, n, j, m);
+                } else {
+                    butterfly<R, false>(v, w, n, j, m);
+                }
+#pragma unroll
+                for (int q = 0; q < R; q++) {
+                    if (out)
+                        p[(b + q * m) * es] = v[q];
+                    else
+                        t[((b + q * m) << LB) + c] = v[q];
+                }
+            }
+        };
+        by_radix<BIG>(r, run);
+        if (!out) __syncthreads();
+    }
+}
+
+__device__ __forceinline__ int padx(int i) { return i + (i >> 3); }  // strides of 8 over all banks
+
+// Rows, real to half spectrum (256^3, 269 MB: 61 us, the library's 56): two rows as the real and the imaginary part of one
+// complex row, separated afterwards. src: the first interior cell of a ghosted
+// array; row q is row (q % ny, q / ny). pairs rows pairs per workgroup.
+template <bool BIG>
+__global__ void __launch_bounds__(FT) k_fft_x(FftDim D, Grid G, const double *__restrict__ src, double2 *__restrict__ dst,
+                                              int nrows, int pairs, int pitch) {
+    extern __shared__ double2 sm[];
+    const int n = D.n, ld = padx(n) + 1, nxh = n / 2 + 1, T = blockDim.x;
+    double2 *w = sm, *t = sm + n;
+    unsigned short *pos = reinterpret_cast<unsigned short *>(t + pairs * ld);
+    for (int i = threadIdx.x; i < n; i += T) {
+        w[i] = D.w[i];
+        pos[i] = D.pos[i];
+    }
+    const int row0 = blockIdx.x * pairs * 2, my = min(pairs, (nrows - row0 + 1) / 2);
+    __syncthreads();
+    for (int k = 0; k < D.np; k++) {
+        const int r = D.r[k], m = D.m[k], ng = n / r;
+        const unsigned magic = D.magic[k];
+        auto run = [&](auto rc) {
+            constexpr int R = decltype(rc)::value;
+            for (int e = threadIdx.x; e < ng * my; e += T) {
+                const int pr = e / ng, g = e - pr * ng;
+                const int l = div_m(g, m, magic), j = g - l * m, b = l * R * m + j;
+                double2 *__restrict__ tl = t + pr * ld;
+                double2 v[R];
+                if (k == 0) {
+                    const int qa = row0 + 2 * pr, qb = qa + 1;
+                    const double *__restrict__ ra = src + ((long long)(qa / G.ny) * G.nyo + qa % G.ny) * G.nxo;
+                    const double *__restrict__ rb = src + ((long long)(qb / G.ny) * G.nyo + qb % G.ny) * G.nxo;
+                    const bool two = qb < nrows;
+#pragma unroll
+                    for (int q = 0; q < R; q++) v[q] = make_double2(ra[b + q * m], two ? rb[b + q * m] : 0.0);
+                } else {
+#pragma unroll
+                    for (int q = 0; q < R; q++) v[q] = tl[padx(b + q * m)];
+                }
+                butterfly<R, false>(v, w, n, j, m);
+#pragma unroll
+                for (int q = 0; q < R; q++) tl[padx(b + q * m)] = v[q];
+            }
+        };
+        by_radix<BIG>(r, run);
+        __syncthreads();
+    }
+    for (int e = threadIdx.x; e < nxh * my; e += T) {
+        const int pr = e / nxh, k = e - pr * nxh;
+        const double2 *__restrict__ tl = t + pr * ld;
+        const double2 a = tl[padx(pos[k])], b = tl[padx(pos[k == 0 ? 0 : n - k])];
+        const long long q = row0 + 2 * pr;
+        dst[q * pitch + k] = make_double2(0.5 * (a.x + b.x), 0.5 * (a.y - b.y));
+        if (q + 1 < nrows) dst[(q + 1) * pitch + k] = make_double2(0.5 * (a.y + b.y), 0.5 * (b.x - a.x));
+    }
+}
+
+// Half spectrum to real rows, the inverse of k_fft_x, into the interior of a
+// ghosted array and, with `images`, into every ghost cell that is a periodic
+// image of it (each ghost width at most the box's length): 256^3: 69 us; the
+// library's transform, a copy into the box and the three ghost passes took
+// 49 + 53 + 16.
+template <bool BIG>
+__global__ void __launch_bounds__(FT) k_fft_xinv(FftDim D, Grid G, const double2 *__restrict__ src, double *__restrict__ dst,
+                                                 int nrows, int pairs, int pitch, int images) {
+    extern __shared__ double2 sm[];
+    const int n = D.n, ld = padx(n) + 1, nxh = n / 2 + 1, T = blockDim.x;
+    double2 *w = sm, *t = sm + n;
+    unsigned short *pos = reinterpret_cast<unsigned short *>(t + pairs * ld);
+    for (int i = threadIdx.x; i < n; i += T) {
+        w[i] = D.w[i];
+        pos[i] = D.pos[i];
+    }
+    const int row0 = blockIdx.x * pairs * 2, my = min(pairs, (nrows - row0 + 1) / 2);
+    __syncthreads();
+    for (int e = threadIdx.x; e < nxh * my; e += T) {
+        const int pr = e / nxh, k = e - pr * nxh;
+        double2 *__restrict__ tl = t + pr * ld;
+        const long long q = row0 + 2 * pr;
+        double2 a = src[q * pitch + k], b = q + 1 < nrows ? src[(q + 1) * pitch + k] : make_double2(0.0, 0.0);
+        // the modes that are their own conjugates are real
+        if (k == 0 || 2 * k == n) a.y = b.y = 0.0;
+        tl[padx(pos[k])] = make_double2(a.x - b.y, a.y + b.x);
+        if (k > 0 && 2 * k != n) tl[padx(pos[n - k])] = make_double2(a.x + b.y, b.x - a.y);
+    }
+    __syncthreads();
+    const long long splane = (long long)G.nxo * G.nyo;
+    for (int k = D.np - 1; k >= 0; k--) {
+        const int r = D.r[k], m = D.m[k], ng = n / r;
+        const unsigned magic = D.magic[k];
+        auto run = [&](auto rc) {
+            constexpr int R = decltype(rc)::value;
+            for (int e = threadIdx.x; e < ng * my; e += T) {
+                const int pr = e / ng, g = e - pr * ng;
+                const int l = div_m(g, m, magic), j = g - l * m, b = l * R * m + j;
+                double2 *__restrict__ tl = t + pr * ld;
+                double2 v[R];
+#pragma unroll
+                for (int q = 0; q < R; q++) v[q] = tl[padx(b + q * m)];
+                butterfly<R, true>(v, w, n, j, m);
+                if (k > 0) {
+#pragma unroll
+                    for (int q = 0; q < R; q++) tl[padx(b + q * m)] = v[q];
+                    continue;
+                }
+                for (int h = 0; h < 2; h++) {
+                    const int qr = row0 + 2 * pr + h;
+                    if (qr >= nrows) break;
+                    const int jy = qr % G.ny, kz = qr / G.ny;
+                    for (int iz = -1; iz <= 1; iz++) {
+                        const int zz = kz + iz * G.nz + G.gz;
+                        if (iz != 0 && (!images || zz < 0 || zz >= G.nzo)) continue;
+                        for (int iy = -1; iy <= 1; iy++) {
+                            const int yy = jy + iy * G.ny + G.gy;
+                            if (iy != 0 && (!images || yy < 0 || yy >= G.nyo)) continue;
+                            double *__restrict__ o = dst + zz * splane + (long long)yy * G.nxo + G.gx;
+#pragma unroll
+                            for (int q = 0; q < R; q++) {
+                                const int x = b + q * m;
+                                const double val = h == 0 ? v[q].x : v[q].y;
+                                o[x] = val;
+                                if (images && x < G.gx) o[x + n] = val;
+                                if (images && x >= n - G.gx) o[x - n] = val;
+                            }
+                        }
+                    }
+                }
+            }
+        };
+        by_radix<BIG>(r, run);
+        __syncthreads();
+    }
+}
+
 int sync_all(hipStream_t s, const Grid &g, double *a) {
     const int per[3] = {g.px, g.py, g.pz}, w[3] = {g.gx, g.gy, g.gz};
     const long long e[3] = {(long long)g.nyo * g.nzo, (long long)g.nxo * g.nzo, (long long)g.nxo * g.nyo};
@@ -197,7 +562,11 @@ struct ngap_fft {
     int nst = 0;
     int device = 0;
     int rank = 0;       // directions with more than one cell
-    long long M = 1;    // complex modes of the half spectrum
+    long long M = 1;    // complex modes of the half spectrum (with padding)
+    int pitch = 1, nxh = 1;    // modes of a row, allocated and in use
+    bool own = false;          // the transforms of this file, else the library's
+    bool images = false;       // the inverse fills the ghosts
+    FftDim D[3]{};             // x, y, z
     hipStream_t s = nullptr;
     hipfftHandle fwd = 0, inv = 0;
     bool have_fwd = false, have_inv = false, setup_done = false;
@@ -252,6 +621,137 @@ int sum_parts(ngap_fft *F, const int *d, long long *out) {
     return 0;
 }
 
+// r_p and m_p of n; false if n has other factors or is too long
+bool factor(int n, FftDim *D) {
+    if (n < 2 || n > FFT_MAX) return false;
+    static const int radix[] = {13, 11, 7, 5, 3};
+    D->n = n;
+    D->np = 0;
+    int rest = n;
+    while (rest % 8 == 0) D->r[D->np++] = 8, rest /= 8;
+    if (rest % 4 == 0) D->r[D->np++] = 4, rest /= 4;
+    if (rest % 2 == 0) D->r[D->np++] = 2, rest /= 2;
+    for (int r : radix)
+        while (rest % r == 0) D->r[D->np++] = r, rest /= r;
+    if (rest != 1) return false;
+    int m = n;
+    for (int p = 0; p < D->np; p++) {
+        m /= D->r[p];
+        D->m[p] = m;
+        D->magic[p] = m > 1 ? (unsigned)(((1ULL << 32) + m - 1) / m) : 0;
+    }
+    return true;
+}
+
+// tables of one direction
+int plan_dim(ngap_fft *F, FftDim *D) {
+    const int n = D->n;
+    std::vector<double2> w(n);
+    std::vector<unsigned short> pos(n);
+    const long double tau = 2.0L * acosl(-1.0L);
+    for (int k = 0; k < n; k++) {
+        w[k] = make_double2((double)cosl(tau * k / n), (double)-sinl(tau * k / n));
+        int f = k, at = 0;
+        for (int p = 0; p < D->np; p++) {
+            at += f % D->r[p] * D->m[p];
+            f /= D->r[p];
+        }
+        pos[k] = (unsigned short)at;
+    }
+    double2 *dw = nullptr;
+    unsigned short *dp = nullptr;
+    int rc = dalloc(F, &dw, n);
+    if (!rc) rc = dalloc(F, &dp, n);
+    if (!rc && (hipMemcpy(dw, w.data(), sizeof(double2) * n, hipMemcpyHostToDevice) != hipSuccess ||
+                hipMemcpy(dp, pos.data(), sizeof(unsigned short) * n, hipMemcpyHostToDevice) != hipSuccess))
+        rc = NGAP_ERR_HIP;
+    D->w = dw;
+    D->pos = dp;
+    return rc;
+}
+
+// Row pairs of a workgroup: about 2048 cells, so that 256 threads have one
+// radix-8 butterfly each, but fewer where that leaves less than two workgroups
+// per CU.
+int row_pairs(const Grid &g) {
+    int pr = std::min(16, std::max(1, 2048 / g.nx));
+    while (pr > 1 && (long long)g.ny * g.nz / (2 * pr) < 512) pr /= 2;
+    return pr;
+}
+int threads_for(int cells) { return std::min(FT, std::max(64, (cells / 8 + 63) / 64 * 64)); }
+size_t row_lds(int n, int pr) { return sizeof(double2) * (n + (size_t)pr * (n + n / 8 + 1)) + sizeof(short) * n; }
+size_t col_lds(int n) { return sizeof(double2) * (n + (size_t)n * LINES); }
+
+bool big(const FftDim &D) {
+    for (int p = 0; p < D.np; p++)
+        if (D.r[p] == 7 || D.r[p] > 8) return true;
+    return false;
+}
+
+void rows_fwd(ngap_fft *F, const double *src, double2 *dst) {
+    const int rows = F->g.ny * F->g.nz, pr = row_pairs(F->g);
+    hipLaunchKernelGGL(big(F->D[0]) ? k_fft_x<true> : k_fft_x<false>, dim3((unsigned)((rows + 2 * pr - 1) / (2 * pr))),
+                       dim3(threads_for(pr * F->g.nx)), row_lds(F->g.nx, pr), F->s, F->D[0], F->g, src, dst, rows, pr, F->pitch);
+}
+
+void rows_inv(ngap_fft *F, const double2 *src, double *dst) {
+    const int rows = F->g.ny * F->g.nz, pr = row_pairs(F->g);
+    hipLaunchKernelGGL(big(F->D[0]) ? k_fft_xinv<true> : k_fft_xinv<false>,
+                       dim3((unsigned)((rows + 2 * pr - 1) / (2 * pr))), dim3(threads_for(pr * F->g.nx)), row_lds(F->g.nx, pr), F->s, F->D[0], F->g,
+                       src, dst, rows, pr, F->pitch, F->images ? 1 : 0);
+}
+
+template <int MODE>
+auto col_kernel(const FftDim &D) {
+    return big(D) ? k_fft_col<MODE, true> : k_fft_col<MODE, false>;
+}
+
+template <int MODE>
+void cols(ngap_fft *F, int ax, double2 *a, double scale) {
+    const Grid &g = F->g;
+    const int n = F->D[ax].n;
+    const long long row = F->pitch, plane = row * g.ny;
+    const int lines = (int)(ax == 1 ? row : plane);
+    hipLaunchKernelGGL(col_kernel<MODE>(F->D[ax]), dim3((unsigned)((lines + LINES - 1) / LINES), ax == 1 ? g.nz : 1),
+                       dim3(threads_for(n * LINES)), col_lds(n), F->s, F->D[ax], (const double2 *)F->d_finv, a, lines,
+                       ax == 1 ? row : plane, plane, F->pitch, F->nxh, scale);
+}
+
+// more than 64 KB of LDS is asked for by name
+bool allow_lds(const FftDim &D) {
+    const int lds = (int)col_lds(D.n);
+    if (lds <= 65536) return true;
+    const void *k[] = {(const void *)col_kernel<FWD>(D), (const void *)col_kernel<INV>(D),
+                       (const void *)col_kernel<DIVIDE>(D)};
+    for (const void *q : k)
+        if (hipFuncSetAttribute(q, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return false;
+    return true;
+}
+
+// own transforms: the operator's spectrum, and a whole solve
+void own_forward(ngap_fft *F, const double *src, double2 *dst) {
+    rows_fwd(F, src, dst);
+    if (F->g.ny > 1) cols<FWD>(F, 1, dst, 1.0);
+    if (F->g.nz > 1) cols<FWD>(F, 2, dst, 1.0);
+}
+
+void own_solve(ngap_fft *F, const double *src, double *dst) {
+    const Grid &g = F->g;
+    const double scale = 1.0 / ((double)g.nx * g.ny * g.nz);
+    rows_fwd(F, src, F->d_spec);
+    if (g.nz > 1) {
+        if (g.ny > 1) cols<FWD>(F, 1, F->d_spec, 1.0);
+        cols<DIVIDE>(F, 2, F->d_spec, scale);
+        if (g.ny > 1) cols<INV>(F, 1, F->d_spec, 1.0);
+    } else if (g.ny > 1) {
+        cols<DIVIDE>(F, 1, F->d_spec, scale);
+    } else {
+        hipLaunchKernelGGL(k_divide, dim3(blocks_for(F->M)), dim3(PT), 0, F->s, F->M, F->d_spec,
+                           (const double2 *)F->d_finv, scale);
+    }
+    rows_inv(F, F->d_spec, dst);
+}
+
 int setup_from(ngap_fft *F, const double *d_opr, double tol) {
     const Grid &g = F->g;
     F->setup_done = false;
@@ -263,7 +763,9 @@ int setup_from(ngap_fft *F, const double *d_opr, double tol) {
     if (bad) return NGAP_ERR_NOT_CIRCULANT;
     hipLaunchKernelGGL(k_zero, dim3(blocks_for(g.No)), dim3(PT), 0, F->s, F->d_kern, g.No);
     hipLaunchKernelGGL(k_place, dim3(1), dim3(64), 0, F->s, g, F->nst, (const int *)F->d_stc, d_opr, F->d_kern);
-    if (F->rank > 0) {
+    if (F->own) {
+        own_forward(F, F->d_kern + F->off, F->d_finv);
+    } else if (F->rank > 0) {
         const hipfftResult r = hipfftExecD2Z(F->fwd, F->d_kern + F->off, (hipfftDoubleComplex *)F->d_finv);
         if (r != HIPFFT_SUCCESS) return fail("hipfftExecD2Z (setup)", (int)r);
     } else if (hipMemcpyAsync(F->d_finv, F->d_kern + F->off, sizeof(double), hipMemcpyDeviceToDevice, F->s) !=
@@ -271,7 +773,8 @@ int setup_from(ngap_fft *F, const double *d_opr, double tol) {
         return NGAP_ERR_HIP;  // one cell: the transform is the value itself (imaginary part set below)
     }
     if (F->rank == 0) hipLaunchKernelGGL(k_zero, dim3(1), dim3(PT), 0, F->s, (double *)F->d_finv + 1, 1LL);
-    hipLaunchKernelGGL(k_invert, dim3(NB), dim3(PT), 0, F->s, F->M, F->d_finv, F->d_part, F->d_part + NB);
+    hipLaunchKernelGGL(k_invert, dim3(NB), dim3(PT), 0, F->s, F->M, F->pitch, F->nxh, F->d_finv, F->d_part,
+                       F->d_part + NB);
     rc = fin(F);
     long long small = 0, nan = 0;
     if (!rc) rc = sum_parts(F, F->d_part, &small);
@@ -285,7 +788,9 @@ int setup_from(ngap_fft *F, const double *d_opr, double tol) {
 int solve_on(ngap_fft *F, const double *d_rhs, double *d_sol) {
     const Grid &g = F->g;
     if (hipEventRecord(F->e0, F->s) != hipSuccess) return fail("hipEventRecord", 0);
-    if (F->rank > 0) {
+    if (F->own) {
+        own_solve(F, d_rhs + F->off, d_sol);
+    } else if (F->rank > 0) {
         // the plans read the interior of rhs and write the interior of sol in place
         hipfftResult r = hipfftExecD2Z(F->fwd, const_cast<double *>(d_rhs) + F->off, (hipfftDoubleComplex *)F->d_spec);
         if (r != HIPFFT_SUCCESS) return fail("hipfftExecD2Z", (int)r);
@@ -297,7 +802,7 @@ int solve_on(ngap_fft *F, const double *d_rhs, double *d_sol) {
     } else {
         hipLaunchKernelGGL(k_zero, dim3(1), dim3(PT), 0, F->s, d_sol + F->off, 1LL);  // the only mode is the zero mode
     }
-    sync_all(F->s, g, d_sol);
+    if (!F->images) sync_all(F->s, g, d_sol);
     if (hipEventRecord(F->e1, F->s) != hipSuccess) return fail("hipEventRecord", 0);
     int rc = fin(F);
     if (rc) return rc;
@@ -352,6 +857,16 @@ int ngap_fft_create(ngap_fft **fp, const ngap_grid *gr, int nst, const int *stc)
     F->M = 1;
     for (int d = 0; d + 1 < r; d++) F->M *= dims[d];
     if (r > 0) F->M *= dims[r - 1] / 2 + 1;
+    F->own = g.nx > 1 && factor(g.nx, &F->D[0]) && (g.ny == 1 || factor(g.ny, &F->D[1])) &&
+             (g.nz == 1 || factor(g.nz, &F->D[2])) && (long long)g.ny * g.nz < (1LL << 30) && g.nz < 65536;
+    if (F->own) {
+        F->nxh = g.nx / 2 + 1;
+        F->pitch = (F->nxh + 7) / 8 * 8;
+        F->M = (long long)F->pitch * g.ny * g.nz;
+        F->images = g.px && g.py && g.pz && g.gx <= g.nx && g.gy <= g.ny && g.gz <= g.nz;
+    } else {
+        F->pitch = F->nxh = r > 0 ? dims[r - 1] / 2 + 1 : 1;
+    }
     // real side: the ghosted array (embed[d] = stride ratio of consecutive
     // directions, the fastest stride as the element stride); complex side: the
     // dense half spectrum
@@ -370,7 +885,11 @@ int ngap_fft_create(ngap_fft **fp, const ngap_grid *gr, int nst, const int *stc)
     if (!rc) rc = dalloc(F, &F->d_spec, (size_t)F->M);
     if (!rc) rc = dalloc(F, &F->d_finv, (size_t)F->M);
     if (!rc && hipMemcpy(F->d_stc, stc, sizeof(int) * 3 * nst, hipMemcpyHostToDevice) != hipSuccess) rc = NGAP_ERR_HIP;
-    if (!rc && r > 0) {
+    for (int d = 0; d < 3 && !rc && F->own; d++) {
+        if (F->D[d].n) rc = plan_dim(F, &F->D[d]);
+        if (!rc && d > 0 && F->D[d].n && !allow_lds(F->D[d])) rc = NGAP_ERR_HIP;
+    }
+    if (!rc && r > 0 && !F->own) {
         if (hipfftPlanMany(&F->fwd, r, dims, rembed, rstride, (int)g.No, cembed, 1, (int)F->M, HIPFFT_D2Z, 1) !=
             HIPFFT_SUCCESS)
             rc = NGAP_ERR_HIP;
