@@ -1170,6 +1170,28 @@ static bool pairs_on(const Geo &g) {
 // mixed: 27.40 against 27.20 ms per solve). Both give the same bits.
 constexpr long long ZSWEEP_MIN_CELLS = 1LL << 20;
 
+// The three transfers below level l as one launch: l + 1 and l + 2 are skipped
+// levels, l + 3 is at most `top`.
+template <typename T>
+struct Skip3 {
+    Geo g[4];
+    int dirs[3];
+    const T *pm[3], *pp[3];
+    bool on = false;
+    Skip3(ngap_t *h, int l, int top) {
+        if (l + 3 > top || h->lev[l + 1].relax || h->lev[l + 2].relax) return;
+        g[0] = h->lev[l].g;
+        for (int i = 0; i < 3; i++) {
+            dirs[i] = h->lev[l + i].cdir;
+            g[i + 1] = h->lev[l + i + 1].g;
+            LevelData<T> &D = data<T>(h->lev[l + i + 1]);
+            pm[i] = D.pm;
+            pp[i] = D.pp;
+        }
+        on = dirs[0] != dirs[1] && dirs[0] != dirs[2] && dirs[1] != dirs[2];
+    }
+};
+
 // One V(nu_pre, nu_post) cycle from a zero guess: v0 = M f0.
 // Sweeps are out of place; on each level the iterate alternates between the
 // level's two buffers so that the last post-smoothing sweep lands in the
@@ -1193,17 +1215,35 @@ void vcycle(ngap_t *h, const T *f0, T *v0) {
     const int lb = bottom_start<T>(h);
     const int top = lb < nl ? lb : nl - 1;  // first level below the per-level loop
     std::vector<T *> pre(nl);
+    std::vector<char> bridged(nl, 0);  // skipped levels that a Skip3 launch passes over
+    auto restrict_from = [&](int l, const T *r) {
+        const Skip3<T> k(h, l, top);
+        if (k.on && launch_gather3<T>(s, k.g, k.dirs, k.pm, k.pp, r, data<T>(h->lev[l + 3]).f)) {
+            bridged[l + 1] = bridged[l + 2] = 1;
+            return;
+        }
+        LevelData<T> &DC = data<T>(h->lev[l + 1]);
+        launch_gather<T>(s, h->lev[l].g, h->lev[l + 1].g, h->lev[l].cdir, r, DC.pm, DC.pp, DC.f);
+    };
+    auto prolong_to = [&](int l, const T *vin, T *vout) {
+        if (l + 1 < nl && bridged[l + 1]) {
+            const Skip3<T> k(h, l, top);
+            launch_prolong3<T>(s, k.g, k.dirs, k.pm, k.pp, data<T>(h->lev[l + 3]).v, vin, vout);
+            return;
+        }
+        LevelData<T> &DC = data<T>(h->lev[l + 1]);
+        launch_prolong_to<T>(s, h->lev[l].g, h->lev[l + 1].g, h->lev[l].cdir, DC.pm, DC.pp, DC.v, vin, vout);
+    };
     for (int l = 0; l < top; l++) {
+        if (bridged[l]) continue;
         Level &L = h->lev[l];
         LevelData<T> &D = data<T>(L);
         const T *f = l == 0 ? f0 : D.f;
         T *fin = l == 0 ? v0 : D.v;
         if (!L.relax) {
             // skipped level: v = 0, so the residual is f; restrict it as it is
-            Level &Cn = h->lev[l + 1];
-            LevelData<T> &DC = data<T>(Cn);
-            launch_gather<T>(s, L.g, Cn.g, L.cdir, f, DC.pm, DC.pp, DC.f);
             pre[l] = nullptr;
+            restrict_from(l, f);
             continue;
         }
         const int npl = post_launches(L), prl = pre_launches(L);
@@ -1230,12 +1270,10 @@ void vcycle(ngap_t *h, const T *f0, T *v0) {
             nb ^= 1;
         }
         pre[l] = const_cast<T *>(cur);
-        Level &Cn = h->lev[l + 1];
-        LevelData<T> &DC = data<T>(Cn);
         // residual into the level's other buffer (free until post-smoothing), then P^T
         T *rbuf = (cur == fin) ? D.w : fin;
         launch_resid<T>(s, L.g, D.c, D.a0, D.a1, D.a2, f, cur, rbuf);
-        launch_gather<T>(s, L.g, Cn.g, L.cdir, rbuf, DC.pm, DC.pp, DC.f);
+        restrict_from(l, rbuf);
     }
     if (lb < nl) {
         launch_bottom_levels<T>(h, lb);
@@ -1245,19 +1283,18 @@ void vcycle(ngap_t *h, const T *f0, T *v0) {
         coarse_solve<T>(h, nl == 1 ? f0 : D.f, nl == 1 ? v0 : D.v);
     }
     for (int l = top - 1; l >= 0; l--) {
+        if (bridged[l]) continue;
         Level &L = h->lev[l];
         LevelData<T> &D = data<T>(L);
         const T *f = l == 0 ? f0 : D.f;
         T *fin = l == 0 ? v0 : D.v;
-        Level &Cn = h->lev[l + 1];
-        LevelData<T> &DC = data<T>(Cn);
         if (!L.relax) {
             // skipped level: v = P v_coarse into the level's final buffer
-            launch_prolong_to<T>(s, L.g, Cn.g, L.cdir, DC.pm, DC.pp, DC.v, (const T *)nullptr, fin);
+            prolong_to(l, nullptr, fin);
             continue;
         }
         T *cur = pre[l];
-        launch_prolong_to<T>(s, L.g, Cn.g, L.cdir, DC.pm, DC.pp, DC.v, cur, cur);
+        prolong_to(l, cur, cur);
         for (int sw = 0; sw < npost;) {
             T *nxt = (cur == fin) ? D.w : fin;
             if (npost - sw >= 2 && pairs_on<T>(L.g)) {

@@ -25,6 +25,15 @@ void launch_apply_x32(hipStream_t s, const Geo &g, const double *c, const double
 template <typename T>
 void launch_sweep(hipStream_t s, const Geo &g, const T *c, const T *a0, const T *a1, const T *a2, const T *f,
                   const T *vin, T *vout, int c1, bool one_cell = false);
+// three transfers in one launch between level g[0] and g[3] (directions dirs[0..2],
+// weights pm, pp of levels 1..3); false, with nothing launched, unless the
+// directions all differ
+template <typename T>
+bool launch_gather3(hipStream_t s, const Geo *g, const int *dirs, const T *const *pm, const T *const *pp, const T *r,
+                    T *fc);
+template <typename T>
+bool launch_prolong3(hipStream_t s, const Geo *g, const int *dirs, const T *const *pm, const T *const *pp,
+                     const T *vc, const T *vin, T *vout);
 // true where launch_sweep2 can take k_sweep2_pair: FP32, even row length, and
 // even counts where periodic (an odd one has no red-black order across the wrap;
 // k_sweep2 colours by the wrapped index). Offsets in a plane are 32 bits of bytes.

@@ -961,6 +961,147 @@ __global__ void __launch_bounds__(SX *SY) k_sweep2(Geo g, const T *__restrict__ 
     }
 }
 
+// ------------------------------------------------------------------ transfers over skipped levels
+// Three transfers along three directions in one launch, between a level and the
+// third one below it when the two levels between are not smoothed (full
+// coarsening): neither is stored. DA, DB, DC: the directions in the order of the
+// coarsening. One thread per cell of the lowest level; per value the operations
+// of k_gather_t and k_prolong_t, so the same bits as three launches.
+// Bound by the latency of the loads and, on large levels, by the intermediate
+// levels' passes that it saves: all loads are unconditional (a value that is not
+// there repeats another and is left out by a select), since behind branches they
+// ran one after the other (13.2 us a restriction). FP64, mean of the cycle's
+// chains on 128^3: three restrictions 11.6 -> 9.9 us, three prolongations 13.7 ->
+// 11.1 us; on 64^3 9.2 -> 4.6 and 13.3 -> 6.5 us.
+template <typename T>
+struct Chain {
+    Geo g[4];                   // the level and the three below
+    const T *pm[3], *pp[3];     // weights, stored on levels 1, 2, 3
+};
+
+template <int DA, int DB>
+__device__ __forceinline__ int at_abc(const Geo &g, int a, int b, int c) {
+    const int x = DA == 0 ? a : (DB == 0 ? b : c), y = DA == 1 ? a : (DB == 1 ? b : c),
+              z = DA == 2 ? a : (DB == 2 ? b : c);
+    return (z * g.n1 + y) * g.n0 + x;
+}
+template <int D>
+__device__ __forceinline__ int len(const Geo &g) {
+    return D == 0 ? g.n0 : (D == 1 ? g.n1 : g.n2);
+}
+template <int D>
+__device__ __forceinline__ int per(const Geo &g) {
+    return D == 0 ? g.p0 : (D == 1 ? g.p1 : g.p2);
+}
+
+// P^T along one direction at coarse position e: v(fine position), the weights'
+// values through w(positions on the coarse level)
+template <int D, typename T, typename V, typename W>
+__device__ __forceinline__ T gather1(const Geo &F, const Geo &C, int e, const T *pm, const T *pp, V v, W w) {
+#pragma clang fp contract(off)
+    const int n = len<D>(F), l = nbm(2 * e, n, per<D>(F)), el = nbm(e, len<D>(C), per<D>(C));
+    const bool odd = 2 * e + 1 < n;
+    const T v0 = v(2 * e), v1 = v(odd ? 2 * e + 1 : 2 * e), vl = v(l >= 0 ? l : 2 * e);
+    const T w0 = pm[w(e)], wl = pp[w(el >= 0 ? el : e)];
+    T s = v0;
+    s = odd ? fma_t(w0, v1, s) : s;
+    s = l >= 0 ? fma_t(wl, vl, s) : s;
+    return s;
+}
+
+template <typename T, int DA, int DB, int DC>
+__global__ void __launch_bounds__(256) k_gather3(Chain<T> ch, const T *__restrict__ r, T *__restrict__ fc) {
+    const Geo g0 = ch.g[0], g1 = ch.g[1], g2 = ch.g[2], g3 = ch.g[3];
+    const T *__restrict__ m1 = ch.pm[0], *__restrict__ p1 = ch.pp[0], *__restrict__ m2 = ch.pm[1],
+            *__restrict__ p2 = ch.pp[1], *__restrict__ m3 = ch.pm[2], *__restrict__ p3 = ch.pp[2];
+    const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y * blockDim.y + threadIdx.y, z = blockIdx.z;
+    if (x >= g3.n0 || y >= g3.n1) return;
+    const int A = DA == 0 ? x : (DA == 1 ? y : z), B = DB == 0 ? x : (DB == 1 ? y : z),
+              C = DC == 0 ? x : (DC == 1 ? y : z);
+    auto v1 = [&](int b, int c) {
+        return gather1<DA>(
+            g0, g1, A, m1, p1, [&](int a) { return r[at_abc<DA, DB>(g0, a, b, c)]; },
+            [&](int a) { return at_abc<DA, DB>(g1, a, b, c); });
+    };
+    auto v2 = [&](int c) {
+        return gather1<DB>(
+            g1, g2, B, m2, p2, [&](int b) { return v1(b, c); }, [&](int b) { return at_abc<DA, DB>(g2, A, b, c); });
+    };
+    fc[(z * g3.n1 + y) * g3.n0 + x] = gather1<DC>(
+        g2, g3, C, m3, p3, [&](int c) { return v2(c); }, [&](int c) { return at_abc<DA, DB>(g3, A, B, c); });
+}
+
+// the odd fine value between two coarse ones (i: the weights' index; right: there is
+// a second one)
+template <typename T>
+__device__ __forceinline__ T between(const T *pm, const T *pp, int i, T v0, T v1, bool right) {
+#pragma clang fp contract(off)
+    const T wm = pm[i], wp = pp[i], add = wm * v0;
+    return right ? fma_t(wp, v1, add) : add;
+}
+
+// vin == nullptr: vout = P v_c
+template <typename T, int DA, int DB, int DC>
+__global__ void __launch_bounds__(256) k_prolong3(Chain<T> ch, const T *__restrict__ vc, const T *vin, T *vout) {
+#pragma clang fp contract(off)
+    const Geo g0 = ch.g[0], g1 = ch.g[1], g2 = ch.g[2], g3 = ch.g[3];
+    const T *__restrict__ m1 = ch.pm[0], *__restrict__ p1 = ch.pp[0], *__restrict__ m2 = ch.pm[1],
+            *__restrict__ p2 = ch.pp[1], *__restrict__ m3 = ch.pm[2], *__restrict__ p3 = ch.pp[2];
+    const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y * blockDim.y + threadIdx.y, z = blockIdx.z;
+    if (x >= g3.n0 || y >= g3.n1) return;
+    const int A = DA == 0 ? x : (DA == 1 ? y : z), B = DB == 0 ? x : (DB == 1 ? y : z),
+              C = DC == 0 ? x : (DC == 1 ? y : z);
+    const int A1 = nbp(A, len<DA>(g3), per<DA>(g3)), B1 = nbp(B, len<DB>(g3), per<DB>(g3)),
+              C1 = nbp(C, len<DC>(g3), per<DC>(g3));
+    const bool ra = A1 >= 0, rb = B1 >= 0, rc = C1 >= 0;
+    const bool oa = 2 * A + 1 < len<DA>(g0), ob = 2 * B + 1 < len<DB>(g0), oc = 2 * C + 1 < len<DC>(g0);
+    const int a_[2] = {A, ra ? A1 : A}, b_[2] = {B, rb ? B1 : B};
+    const int c1 = rc ? C1 : C;
+    // along DC: level 2 at (a_, b_, 2C + 0, 1); a skipped level's value is 0 + P v
+    T t2[2][2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int at = at_abc<DA, DB>(g3, a_[i], b_[j], C);
+            const T u0 = vc[at], u1 = vc[at_abc<DA, DB>(g3, a_[i], b_[j], c1)];
+            t2[i][j][0] = T(0) + u0;
+            t2[i][j][1] = T(0) + between(m3, p3, at, u0, u1, rc);
+        }
+    // along DB: level 1 at (a_, 2B + 0, 1, 2C + 0, 1)
+    T t1[2][2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            t1[i][0][k] = T(0) + t2[i][0][k];
+            t1[i][1][k] = T(0) + between(m2, p2, at_abc<DA, DB>(g2, a_[i], B, k && oc ? 2 * C + 1 : 2 * C), t2[i][0][k],
+                                         t2[i][1][k], rb);
+        }
+    // along DA: this level (a cell past an odd end repeats the one before it)
+    T o[2][2][2], w[2][2][2];
+    int ao[2][2][2];
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int fb = j && ob ? 2 * B + 1 : 2 * B, fc = k && oc ? 2 * C + 1 : 2 * C;
+            ao[0][j][k] = at_abc<DA, DB>(g0, 2 * A, fb, fc);
+            ao[1][j][k] = at_abc<DA, DB>(g0, oa ? 2 * A + 1 : 2 * A, fb, fc);
+            o[0][j][k] = t1[0][j][k];
+            o[1][j][k] = between(m1, p1, at_abc<DA, DB>(g1, A, fb, fc), t1[0][j][k], t1[1][j][k], ra);
+#pragma unroll
+            for (int i = 0; i < 2; i++) w[i][j][k] = vin ? vin[ao[i][j][k]] : T(0);
+        }
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                if ((!i || oa) && (!j || ob) && (!k || oc)) vout[ao[i][j][k]] = w[i][j][k] + o[i][j][k];
+}
+
 // ------------------------------------------------------------------ the pair, two cells per lane
 // The pair of k_sweep2 in FP32 on levels of an even row length. In k_sweep2 a
 // lane holds one cell column and half of the lanes idle: at the step whose
@@ -2033,6 +2174,46 @@ void launch_prolong_to(hipStream_t s, const Geo &F, const Geo &C, int d, const T
         hipLaunchKernelGGL((k_prolong_t<T, 2>), grid, dim3(tx, ty), 0, s, F, C, pm, pp, vc, vin, vout);
 }
 
+// directions of a chain: -1 unless all three differ
+static int chain_order(const int *d) { return d[0] != d[1] && d[0] != d[2] && d[1] != d[2] ? 3 * d[0] + d[1] : -1; }
+
+template <typename T, typename F>
+static bool launch_chain(const Geo *g, const int *dirs, const T *const *pm, const T *const *pp, F launch) {
+    Chain<T> ch;
+    for (int i = 0; i < 4; i++) ch.g[i] = g[i];
+    for (int i = 0; i < 3; i++) ch.pm[i] = pm[i], ch.pp[i] = pp[i];
+    // one wave per workgroup: the lowest level is small
+    const int tx = std::min(64, pow2ceil(g[3].n0)), ty = 64 / tx;
+    const dim3 grid((g[3].n0 + tx - 1) / tx, (g[3].n1 + ty - 1) / ty, g[3].n2), block(tx, ty);
+    using std::integral_constant;
+    switch (chain_order(dirs)) {
+        case 1: launch(ch, grid, block, integral_constant<int, 0>(), integral_constant<int, 1>(), integral_constant<int, 2>()); break;
+        case 2: launch(ch, grid, block, integral_constant<int, 0>(), integral_constant<int, 2>(), integral_constant<int, 1>()); break;
+        case 3: launch(ch, grid, block, integral_constant<int, 1>(), integral_constant<int, 0>(), integral_constant<int, 2>()); break;
+        case 5: launch(ch, grid, block, integral_constant<int, 1>(), integral_constant<int, 2>(), integral_constant<int, 0>()); break;
+        case 6: launch(ch, grid, block, integral_constant<int, 2>(), integral_constant<int, 0>(), integral_constant<int, 1>()); break;
+        case 7: launch(ch, grid, block, integral_constant<int, 2>(), integral_constant<int, 1>(), integral_constant<int, 0>()); break;
+        default: return false;
+    }
+    return true;
+}
+
+template <typename T>
+bool launch_gather3(hipStream_t s, const Geo *g, const int *dirs, const T *const *pm, const T *const *pp, const T *r,
+                    T *fc) {
+    return launch_chain<T>(g, dirs, pm, pp, [&](const Chain<T> &ch, dim3 grid, dim3 block, auto a, auto b, auto c) {
+        hipLaunchKernelGGL((k_gather3<T, a(), b(), c()>), grid, block, 0, s, ch, r, fc);
+    });
+}
+
+template <typename T>
+bool launch_prolong3(hipStream_t s, const Geo *g, const int *dirs, const T *const *pm, const T *const *pp,
+                     const T *vc, const T *vin, T *vout) {
+    return launch_chain<T>(g, dirs, pm, pp, [&](const Chain<T> &ch, dim3 grid, dim3 block, auto a, auto b, auto c) {
+        hipLaunchKernelGGL((k_prolong3<T, a(), b(), c()>), grid, block, 0, s, ch, vc, vin, vout);
+    });
+}
+
 template <typename Tin, typename Tout>
 void launch_dense(hipStream_t s, int n, const double *Ainv, const Tin *f, Tout *v) {
     hipLaunchKernelGGL((k_dense_t<Tin, Tout>), dim3((n + 3) / 4), dim3(256), 0, s, n, Ainv, f, v);
@@ -2058,6 +2239,10 @@ template void launch_bottom<float>(hipStream_t, const BotArgs<float> &);
                                    T *, bool);                                                                     \
     template void launch_prolong_to<T>(hipStream_t, const Geo &, const Geo &, int, const T *, const T *,           \
                                        const T *, const T *, T *, bool);                                           \
+    template bool launch_gather3<T>(hipStream_t, const Geo *, const int *, const T *const *, const T *const *,     \
+                                    const T *, T *);                                                               \
+    template bool launch_prolong3<T>(hipStream_t, const Geo *, const int *, const T *const *, const T *const *,    \
+                                     const T *, const T *, T *);                                                   \
     template void launch_dense<T, T>(hipStream_t, int, const double *, const T *, T *);
 INST(double)
 INST(float)
