@@ -28,6 +28,9 @@ long long ngapnet_small_wgrad_part_size(int cout);
 int ngapnet_relu_bwd(const float *dy, const void *y_bf16, float *dx, void *dxb_bf16, long long n, void *stream);
 int ngapnet_to_bf16(const float *s, void *d_bf16, long long n, void *stream);
 int ngapnet_pool2(const void *in_bf16, void *out_bf16, int nx, int ny, int nz, int c, void *stream);
+/* The pool, and its input into channels d0 .. d0 + c of a buffer of ctot channels. */
+int ngapnet_pool2_cat(const void *in_bf16, void *out_bf16, void *cat_bf16, int nx, int ny, int nz, int c, int ctot,
+                      int d0, void *stream);
 int ngapnet_pool2_bwd(const float *dout, float *din, int nx, int ny, int nz, int c, int acc, void *stream);
 int ngapnet_up2(const void *in_bf16, void *out_bf16, int nx, int ny, int nz, int c, int ctot, int c0, void *stream);
 int ngapnet_up2_bwd(const float *dout, float *din, int nx, int ny, int nz, int c, int ctot, int c0, void *stream);

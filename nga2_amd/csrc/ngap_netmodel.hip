@@ -185,22 +185,19 @@ int forward(ngapnet *M, hipStream_t s) {
     const long long *V = M->V;
     int(*S)[3] = M->shp;
     NCK(ngapnet_conv3_small_fwd(M->x, M->w32 + M->off[C0], nullptr, M->c0, S[0][0], S[0][1], S[0][2], 1, 32, 1, s));
-    NCK(ngapnet_pool2(M->c0, M->p1, S[0][0], S[0][1], S[0][2], 32, s));
+    NCK(ngapnet_pool2_cat(M->c0, M->p1, M->cat0, S[0][0], S[0][1], S[0][2], 32, 64, 32, s));
     NCK(conv(M, C1, M->p1, M->c1, s));
-    NCK(ngapnet_pool2(M->c1, M->p2, S[1][0], S[1][1], S[1][2], 32, s));
+    NCK(ngapnet_pool2_cat(M->c1, M->p2, M->cat1, S[1][0], S[1][1], S[1][2], 32, 96, 64, s));
     NCK(conv(M, C2A, M->p2, M->c2a, s));
     NCK(conv(M, C2, M->c2a, M->c2, s));
-    NCK(ngapnet_pool2(M->c2, M->p3, S[2][0], S[2][1], S[2][2], 64, s));
+    NCK(ngapnet_pool2_cat(M->c2, M->p3, M->cat2, S[2][0], S[2][1], S[2][2], 64, 128, 64, s));
     NCK(conv(M, B1, M->p3, M->b1, s));
     NCK(conv(M, B, M->b1, M->b, s));
     NCK(ngapnet_up2(M->b, M->cat2, S[2][0], S[2][1], S[2][2], 64, 128, 0, s));
-    NCK(ngapnet_chan_copy_bf16(M->c2, M->cat2, V[2], 64, 64, 0, 128, 64, s));
     NCK(conv(M, D2, M->cat2, M->d2, s));
     NCK(ngapnet_up2(M->d2, M->cat1, S[1][0], S[1][1], S[1][2], 64, 96, 0, s));
-    NCK(ngapnet_chan_copy_bf16(M->c1, M->cat1, V[1], 32, 32, 0, 96, 64, s));
     NCK(conv(M, D1, M->cat1, M->d1, s));
     NCK(ngapnet_up2(M->d1, M->cat0, S[0][0], S[0][1], S[0][2], 32, 64, 0, s));
-    NCK(ngapnet_chan_copy_bf16(M->c0, M->cat0, V[0], 32, 32, 0, 64, 32, s));
     NCK(conv(M, D0, M->cat0, M->d0, s));
     NCK(ngapnet_conv1_fwd(M->d0, M->w32 + M->off[OUT], M->y, V[0], 32, s));
     return 0;

@@ -59,6 +59,7 @@ def lib():
         L.ngapnet_relu_bwd.argtypes = [_vp, _vp, _vp, _vp, _ll, _vp]
         L.ngapnet_to_bf16.argtypes = [_vp, _vp, _ll, _vp]
         L.ngapnet_pool2.argtypes = [_vp, _vp, _i, _i, _i, _i, _vp]
+        L.ngapnet_pool2_cat.argtypes = [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp]
         L.ngapnet_pool2_bwd.argtypes = [_vp, _vp, _i, _i, _i, _i, _i, _vp]
         L.ngapnet_up2.argtypes = [_vp, _vp, _i, _i, _i, _i, _i, _i, _vp]
         L.ngapnet_up2_bwd.argtypes = [_vp, _vp, _i, _i, _i, _i, _i, _i, _vp]
