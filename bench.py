@@ -753,7 +753,7 @@ def main():
         host_res = host_path_leg(args, P, 1e3 * mixed["elapsed"] / args.steps)
 
     # Roofline of the kernel that runs on the fine level of the headline (mixed) cycle: its
-    # post-smoothing pair k_sweep2<float,16,false>, the largest fine-level launch. "achieved"
+    # post-smoothing pair k_sweep2_pair<false>, the largest fine-level launch. "achieved"
     # counts the algorithmic bytes of its one pass over the arrays (7 x 4 B per cell);
     # "sweep_equiv_gbs" the bytes of the two single-sweep launches it replaces. The other
     # fine-level kernels, the single sweep k_sweep<float> (timed on the fine level; in the cycle
@@ -779,13 +779,13 @@ def main():
         return e
 
     post = entry(p2_ms, p2_bytes, "sweep2_post_fp32_channel256.txt",
-                 "k_sweep2<float,16,false>: the fine level's two post-smoothing red/black GS sweeps in one pass",
+                 "k_sweep2_pair<false>: the fine level's two post-smoothing red/black GS sweeps in one pass",
                  2 * rb_bytes)
     roofline = {"bound": "hbm", "achieved": post["achieved"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": post["frac"], "traffic": post["traffic"]}
     roofline.update({k: v for k, v in post.items() if k not in roofline})
     roofline["sweep2_zero_fp32"] = entry(p0_ms, p0_bytes, "sweep2_pre_fp32_channel256.txt",
-                                         "k_sweep2<float,16,true>: the fine level's pre-smoothing pair from a zero iterate",
+                                         "k_sweep2_pair<true>: the fine level's pre-smoothing pair from a zero iterate",
                                          6.0 / 7.0 * rb_bytes + rb_bytes)
     roofline["sweep_fp32"] = entry(rb_ms, rb_bytes, "sweep_fp32_channel256.txt",
                                    "k_sweep<float>: one fused red/black GS sweep (64 x 16 tiles), on the fine level")
