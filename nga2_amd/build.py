@@ -1,5 +1,5 @@
-"""Build recipes: the HIP solver library (gfx950), the CPU oracle used as the
-checker, and the Fortran ``linsol`` shim.
+"""Build recipes: the HIP solver library (gfx950), the CPU oracle that the tests take as the
+reference, and the Fortran ``linsol`` shim.
 
 Everything is built in-tree so the shared objects travel with the source tree.
 """

@@ -1129,9 +1129,10 @@ __global__ void __launch_bounds__(256) k_prolong3(Chain<T> ch, const T *__restri
 // - Six steps per loop iteration: the life of a loaded value, so that the queues
 //   shift by renaming (a copy of a load in flight waits for it), and of the
 //   LDS slots, so that their addresses are constants.
-// Of the 142 us, the loads with their halos take about 110 at 5.5 TB/s, the
-// vector instructions about 60. Per cell the operations and roundings of k_sweep2, so bit-identical to it.
-// 256^3: 247 -> 145 us, from zero 209 -> 142 us.
+// Bound by the traffic of the tiles with their rings: 657 MB a launch by the
+// counters (1.4 times the arrays) at 4.6 TB/s. Per cell the operations and
+// roundings of k_sweep2, so bit-identical to it. In a 256^3 solve 247 -> 145 us,
+// from zero 209 -> 142 us.
 constexpr int PX = 64, PY = 32, PR = 4;
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
@@ -2095,10 +2096,10 @@ void launch_sweep(hipStream_t s, const Geo &g, const T *c, const T *a0, const T 
 }
 
 // Two sweeps of colour order c1 in one launch: k_sweep2_pair where it can run
-// (247 -> 145 us at 256^3), else k_sweep2, 58 x 10 output
-// tiles, about 512 workgroups, z chunks of >= 16 planes on large levels (each
-// chunk recomputes 6 planes). vin and vout must differ; vin == nullptr: the
-// first sweep starts from a zero iterate.
+// (247 -> 145 us at 256^3), else k_sweep2 with 58 x 10 output tiles, about 512
+// workgroups and z chunks of >= 16 planes on large levels (each chunk recomputes
+// 6 planes). vin and vout must differ; vin == nullptr: the first sweep starts
+// from a zero iterate.
 template <typename T>
 void launch_sweep2(hipStream_t s, const Geo &g, const T *c, const T *a0, const T *a1, const T *a2, const T *f,
                    const T *vin, T *vout, int c1, bool one_cell) {
