@@ -950,13 +950,19 @@ int chan_copy(const T *src, T *dst, long long nv, int c, int cs, int s0, int cd,
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
+// boxes and channel counts that the tiled convolutions take
+bool tiled(int nx, int ny, int nz, int cin, int cout) {
+    return nx > 0 && ny > 0 && nz > 0 && cin > 0 && cout > 0 && nx % TXV == 0 && ny % TYV == 0 && nz % TZV == 0 &&
+           cin % CK == 0 && cout % CK == 0;
+}
+
 }  // namespace
 
 extern "C" {
 
 int ngapnet_conv3_fwd(const void *in, const void *wt, float *out32, void *outb, int nx, int ny, int nz, int cin,
                       int cout, int relu, void *stream) {
-    if (cin % CK || cout % CK || nx % TXV || ny % TYV || nz % TZV || cin <= 0 || cout <= 0) return -1;
+    if (!tiled(nx, ny, nz, cin, cout)) return -1;
     const int vst = (uintptr_t)out32 % 16 == 0 && (uintptr_t)outb % 8 == 0;
     const long long wg4 = (long long)(nx / TXV) * (ny / TYV) * (nz / TZV) * (cout / CK);
     // 16 x 8 x 4 tiles where they still give every CU a workgroup; smaller
@@ -988,7 +994,7 @@ int ngapnet_wgrad_parts(int nx, int ny, int nz, int cin, int cout) {
 
 int ngapnet_conv3_wgrad(const void *in, const void *dout, float *dw, float *part, int nx, int ny, int nz, int cin,
                         int cout, void *stream) {
-    if (cin % CK || cout % CK || nx % TXV || ny % TYV || nz % TZV) return -1;
+    if (!tiled(nx, ny, nz, cin, cout)) return -1;
     const int blocks = (cin / CK) * (cout / CK);
     const int wx = nx % 32 == 0 ? 32 : 16;
     const int cols = (nx / wx) * (ny / WY);

@@ -4,6 +4,8 @@ invariants of NGA2's formulas. No kernel is launched here."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -41,6 +43,22 @@ def test_net_library_exports_all_declared_symbols():
     # pure host query: voxel-tile groups of the weight-gradient split
     assert L.ngapnet_wgrad_parts(16, 4, 4, 32, 32) == 1
     assert L.ngapnet_wgrad_parts(256, 256, 256, 32, 32) == 256
+
+
+@pytest.mark.parametrize("call", ["conv3_fwd", "conv3_wgrad"])
+@pytest.mark.parametrize("dims", [(0, 4, 4, 32, 32), (16, 0, 4, 32, 32), (16, 4, 0, 32, 32), (16, 4, 4, 0, 32),
+                                  (16, 4, 4, 32, 0), (16, 4, 4, -32, 32), (-16, -4, 4, 32, 32), (16, 4, 4, 16, 32),
+                                  (24, 4, 4, 32, 32)])
+def test_tiled_convolutions_refuse_empty_and_ragged_boxes(call, dims):
+    """Counts that are zero, negative or no multiple of a tile are refused with
+    a code before anything is computed from them or launched (in a child
+    process: a division by zero on the host would end it)."""
+    n = 4 if call == "conv3_wgrad" else 5
+    code = (f"from nga2_amd import unet; L = unet.lib(); "
+            f"print('RC', L.ngapnet_{call}(*[None] * 4, *{dims}, *[0] * {n - 4}, None))")
+    p = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert p.returncode == 0, p.returncode
+    assert p.stdout.split()[-1] == "-1", p.stdout
 
 
 def test_strerror_and_defaults_without_gpu():
