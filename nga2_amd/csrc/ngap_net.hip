@@ -48,17 +48,22 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 // With one LDS read per tap and operand the kernel was bound by the LDS read
 // rate and by the staging between barriers. So a halo row is read once per
 // (dz, dx) and used for the three taps dy of three output rows (TY + 2 reads
-// for 6 TY MFMAs); the weights do not pass through LDS: each wave loads its six
-// operands of the next (dz, dx) from L1/L2 while it works on this one; and a
-// workgroup walks over several tiles, with the next tile's (or chunk's) halo
-// on its way to registers behind the products. TY = 8 takes 69 KB of LDS: two
-// workgroups per CU. The sched_barriers keep the loads where they are written;
-// the scheduler sinks them to their first use otherwise. D is transposed
-// (weights as the first operand): a lane then holds four consecutive channels
-// of a voxel and stores 8 (BF16) or 16 (FP32) bytes.
-// 64 -> 32 channels at 128^3: 405 us (572 TFLOP/s) with 16 x 4 x 4 tiles and
-// the weights staged in LDS, 312 us (743 TFLOP/s) now; 32 -> 64: 409 to 230 us
-// (1010 TFLOP/s).
+// for 6 TY MFMAs); the weights do not pass through LDS: each wave holds the nine
+// taps of a plane dz and loads the next plane's from L1/L2, each into the
+// registers of a tap that has done its last output row; and a workgroup walks
+// over several tiles, with the next tile's (or chunk's) halo on its way to
+// registers behind the products. TY = 8 takes 69 KB of LDS and 253 registers:
+// two workgroups per CU. The sched_barriers keep the loads where they are
+// written; the scheduler sinks them to their first use otherwise. D is
+// transposed (weights as the first operand): a lane then holds four consecutive
+// channels of a voxel and stores 8 (BF16) or 16 (FP32) bytes.
+// An output sums its taps by chunk, dz, dy, dx. (With dy innermost, six taps of
+// weights would do, and the figures below are 2 to 5% less; but another order
+// flips the BF16 rounding of an output now and then, which a network's later
+// layers turn into 3e-3 of its result.)
+// 64 -> 32 channels at 128^3: 357 us (650 TFLOP/s) with 16 x 4 x 4 tiles and
+// the weights staged in LDS, 266 us (870 TFLOP/s) now; 32 -> 64: 428 to 240 us
+// (970 TFLOP/s). BF16 out, back to back.
 // OFF: the type of a lane's byte offset within a plane of the input (32 bits
 // unless a plane is 4 GB or more), added to an address held in scalar registers.
 template <int TY, typename OFF>
@@ -113,18 +118,16 @@ __global__ void __launch_bounds__(256, 2) k_conv3_fwd(const __bf16 *__restrict__
     };
     const long long wtap = (long long)cout * cin;
     const unsigned wo = (unsigned)(lr * cin + lg * 8) * 2u;
-    bf16x8 w[2][3][2];
-    // weights of group g = (dz, dx): taps dy = 0, 1, 2, two blocks of 16
-    // channels, from the block's (uniform) address wu
-    auto wload = [&](int g, const __bf16 *wu, bf16x8 (&d)[3][2]) {
-        const int dz = g / 3, dx = g - 3 * dz;
+    bf16x8 w[3][3][2];
+    // weights of tap (dz, dy, dx), two blocks of 16 channels, from the chunk's
+    // (uniform) address wu
+    auto wload = [&](const __bf16 *wu, int dz, int dy, int dx) {
 #pragma unroll
-        for (int dy = 0; dy < 3; dy++)
-#pragma unroll
-            for (int mb = 0; mb < 2; mb++)
-                d[dy][mb] = *reinterpret_cast<const bf16x8 *>(
-                    reinterpret_cast<const char *>(wu + (dz * 9 + dy * 3 + dx) * wtap + (long long)mb * 16 * cin) + wo);
+        for (int mb = 0; mb < 2; mb++)
+            w[dy][dx][mb] = *reinterpret_cast<const bf16x8 *>(
+                reinterpret_cast<const char *>(wu + (dz * 9 + dy * 3 + dx) * wtap + (long long)mb * 16 * cin) + wo);
     };
+    auto chunk = [&](int t, int ci0) { return wt + (long long)(t % nco) * CK * cin + ci0; };
     f32x4 acc[TY][2];
     // one pass of the loop per 32-channel chunk of a tile: (t, ci0), then (tn, cn)
     int tn = tfirst, cn = 0;
@@ -132,6 +135,8 @@ __global__ void __launch_bounds__(256, 2) k_conv3_fwd(const __bf16 *__restrict__
         const int z0 = aim(tn);
 #pragma unroll
         for (int hz = 0; hz < HZ; hz++) fetch(z0, cn, hz);
+#pragma unroll
+        for (int dx = 0; dx < 3; dx++) wload(chunk(tn, cn), 0, 0, dx);
     }
     while (tn < tend) {
         const int t = tn, ci0 = cn;
@@ -148,41 +153,50 @@ __global__ void __launch_bounds__(256, 2) k_conv3_fwd(const __bf16 *__restrict__
 #pragma unroll
                 for (int b = 0; b < 2; b++) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
-        const __bf16 *wu = wt + (long long)co0 * cin + ci0;
-        wload(0, wu, w[0]);
+        const int tc = min(tn, tend - 1);  // (behind the last chunk in vain)
+        const __bf16 *wu = chunk(t, ci0), *wn = chunk(tc, cn);
+        // (dy = 0 came with the previous chunk; more taps there, or none, measured slower)
+#pragma unroll
+        for (int q = 3; q < 9; q++) wload(wu, 0, q / 3, q % 3);
         __syncthreads();  // the previous chunk has been read
 #pragma unroll
         for (int hz = 0; hz < HZ; hz++)
 #pragma unroll
             for (int i = 0; i < NL; i++) *reinterpret_cast<u32x4 *>(s_in + hz * PL + lx[i]) = rx[hz][i];
         __syncthreads();
-        const int zn = aim(min(tn, tend - 1));  // (behind the last chunk in vain)
+        const int zn = aim(tc);
+        const __bf16 *base = s_in + PL * wave;
 #pragma unroll
-        for (int g = 0; g < 9; g++) {
-            const int dz = g / 3, dx = g % 3;
-            // one plane of the next chunk per group, behind the next weights:
-            // loads return in order, so the wait for those does not reach it
-            if (g < 8) wload(g + 1, wu, w[(g + 1) & 1]);
-            __builtin_amdgcn_sched_barrier(0);
-            if (g < HZ) fetch(zn, cn, g);
-            const __bf16 *base = s_in + PL * (wave + dz) + xo[dx];
+        for (int dz = 0; dz < 3; dz++) {
             bf16x8 a[3];
-            a[0] = *reinterpret_cast<const bf16x8 *>(base);
-            a[1] = *reinterpret_cast<const bf16x8 *>(base + ROW);
+            a[0] = *reinterpret_cast<const bf16x8 *>(base + dz * PL + xo[0]);
+            a[1] = *reinterpret_cast<const bf16x8 *>(base + dz * PL + xo[1]);
 #pragma unroll
             for (int r = 0; r < HY; r++) {
-                if (r + 2 < HY) a[(r + 2) % 3] = *reinterpret_cast<const bf16x8 *>(base + (r + 2) * ROW);
-                __builtin_amdgcn_sched_barrier(0);
+                if (r == 2) fetch(zn, cn, 2 * dz);
+                if (r == 4) fetch(zn, cn, 2 * dz + 1);
 #pragma unroll
-                for (int dy = 0; dy < 3; dy++) {
-                    const int o = r - dy;
-                    if (o < 0 || o >= TY) continue;
+                for (int dx = 0; dx < 3; dx++) {
+                    const int n = (dx + 2) % 3, rn = r + (dx + 2) / 3;  // two operands ahead
+                    if (rn < HY) a[n] = *reinterpret_cast<const bf16x8 *>(base + dz * PL + rn * ROW + xo[n]);
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int mb = 0; mb < 2; mb++)
-                        acc[o][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[g & 1][dy][mb], a[r % 3], acc[o][mb], 0,
-                                                                             0, 0);
+                    for (int dy = 0; dy < 3; dy++) {
+                        const int o = r - dy;
+                        if (o < 0 || o >= TY) continue;
+#pragma unroll
+                        for (int mb = 0; mb < 2; mb++)
+                            acc[o][mb] =
+                                __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[dy][dx][mb], a[dx], acc[o][mb], 0, 0, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    // a tap that has done its last output row: the next plane's in its place
+                    // (behind the last plane, the next chunk's first three)
+                    if (dz < 2 ? r >= TY - 1 : r == TY - 1) {
+                        wload(dz < 2 ? wu : wn, (dz + 1) % 3, r - (TY - 1), dx);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
                 }
-                __builtin_amdgcn_sched_barrier(0);
             }
         }
         if (ci0 + CK < cin) continue;

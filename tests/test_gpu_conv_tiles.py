@@ -74,3 +74,34 @@ def test_forward_and_weight_gradient(shape, cin, cout, shift):
     dref = torch.stack([g64.T @ _shifted(x64, shape, t) for t in range(27)])
     err = (dw.double().reshape(27, cout, cin) - dref).abs().max() / dref.abs().max()
     assert float(err) <= 2e-5, float(err)
+
+
+@pytest.mark.parametrize("shape,cin", [((16, 4, 4), 32), ((16, 4, 8), 96), ((64, 64, 64), 64)])
+def test_forward_sums_in_order(shape, cin):
+    """An output sums its taps in FP32 by channel chunk, dz, dy, dx: another
+    order would round elsewhere and, through BF16 outputs, change a network's
+    results. One weight of each (chunk, tap) is +-2^24 or +-1 and the input is
+    1, so that every tap adds one number and the sum depends on the order."""
+    from nga2_amd import unet
+
+    L = unet.lib()
+    print(f"\n[conv order {shape} {cin}]", flush=True)
+    cout, chunks = 32, cin // 32
+    gen = torch.Generator(device="cpu").manual_seed(11)
+    val = torch.tensor([2.0 ** 24, -(2.0 ** 24), 1.0, -1.0])[torch.randint(4, (chunks, 27, cout), generator=gen)]
+    at = torch.randint(32, (chunks, 27, cout, 1), generator=gen)
+    w = torch.zeros(chunks, 27, cout, 32).scatter_(3, at, val[..., None])
+    w = w.permute(1, 2, 0, 3).reshape(27, cout, cin).to(torch.bfloat16).contiguous().to(DEV)
+    want = torch.zeros(cout)
+    for c in range(chunks):
+        for t in range(27):
+            want = want + val[c, t]
+    assert not torch.equal(want, val.double().sum((0, 1)).float())
+    V = shape[0] * shape[1] * shape[2]
+    x = torch.ones(V, cin, dtype=torch.bfloat16, device=DEV)
+    out = torch.zeros(V, cout, device=DEV)
+    unet._enter()
+    rc = L.ngapnet_conv3_fwd(_p(x), _p(w), _p(out), None, *shape, cin, cout, 0, None)
+    unet._leave()
+    assert rc == 0
+    assert torch.equal(out.cpu(), want.expand(V, cout))
