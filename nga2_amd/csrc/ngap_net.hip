@@ -12,6 +12,7 @@
 // layer (1-2 input channels) and the 1x1 output layer use plain FP32 kernels.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "ngapnet.h"
@@ -1012,18 +1013,30 @@ int ngapnet_conv3_wgrad(const void *in, const void *dout, float *dw, float *part
     const int blocks = (cin / CK) * (cout / CK);
     const int wx = nx % 32 == 0 ? 32 : 16;
     const int cols = (nx / wx) * (ny / WY);
-    // workgroups per 32 x 32 channel block: two per CU over all blocks, at most
-    // the caller's partials; columns are cut into ranges of planes (at least 4:
-    // each range reads two more) until there is a unit for each
-    int P = ngapnet_wgrad_parts(nx, ny, nz, cin, cout);
-    if (P > 512 / blocks) P = 512 / blocks;
-    if (P < 1) P = 1;
-    int nseg = (P + cols - 1) / cols;
-    if (nseg > nz / 4) nseg = nz / 4;
+    const int G = ngapnet_wgrad_parts(nx, ny, nz, cin, cout);
+    // workgroups per 32 x 32 channel block: two per CU over all blocks; columns
+    // are cut into ranges of planes (at least 4: each range reads two more) until
+    // there is a unit for each
+    const int W = std::max(1, std::min(G, 512 / blocks));
+    int nseg = std::min((W + cols - 1) / cols, nz / 4);
+    // ... and into shorter ranges where a partial would be a longer chain of FP32
+    // sums than 256 partials need. The 2-norm error of dW is about
+    // 2^-24 sqrt(L / 4 + G / 11) for G partials of L products of 32 voxels added
+    // one after the other; here those are added in four slices, so that L may be
+    // G / 4 more. Against 64 bits, with 256 partials, with one per workgroup (the
+    // fewer the more channel blocks), and now: 64^3, 128 -> 128 channels 3.2e-7,
+    // 4.8e-7 (185 us), 2.7e-7 (250 us); 128^3, 96 -> 32 5.7e-7, 6.8e-7 (340 us),
+    // 5.1e-7 (300 us).
+    const long long tiles = (long long)(nx / TXV) * (ny / TYV) * (nz / TZV);
+    const long long most = 256 * ((tiles + G - 1) / G) + 8LL * G;  // voxels of a partial
+    const int zmax = (int)std::max(1LL, std::min((long long)nz, most / (WY * wx)));
+    nseg = std::max(nseg, (nz + zmax - 1) / zmax);
     const int zseg = (nz + nseg - 1) / nseg;
     nseg = (nz + zseg - 1) / zseg;
     const int units = cols * nseg;
-    if (P > units) P = units;
+    // units of a partial; more partials than W run as further workgroups
+    const int each = (int)std::max(1LL, most / ((long long)zseg * WY * wx));
+    const int P = std::min(std::min(G, units), std::max(W, (units + each - 1) / each));
     const dim3 grid((unsigned)(P * blocks));
     if (wx == 32)
         hipLaunchKernelGGL(k_conv3_wgrad<32>, grid, dim3(256), 0, (hipStream_t)stream, (const __bf16 *)in,

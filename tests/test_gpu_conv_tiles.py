@@ -105,3 +105,38 @@ def test_forward_sums_in_order(shape, cin):
     unet._leave()
     assert rc == 0
     assert torch.equal(out.cpu(), want.expand(V, cout))
+
+
+@pytest.mark.parametrize("n,cin,cout", [((64, 64, 64), 128, 128), ((32, 32, 32), 256, 256), ((128, 128, 128), 96, 32)])
+def test_weight_gradient_sums_stay_short(n, cin, cout):
+    """Many channel blocks leave few workgroups per block; the sums of each must
+    not get longer for it. n additions of terms of random sign leave an error of
+    0.41 x 2^-24 of the sum at each, 2^-24 sqrt(n / 12) in all; the matrix unit's
+    own additions round worse (measured: sqrt(n / 4)). The bound is that of L
+    products of 32 voxels each in at most 256 partials, and their sum one by
+    one, with n / 8 and L / 3.5 for margin."""
+    from nga2_amd import unet
+
+    L = unet.lib()
+    print(f"\n[conv wgrad sums {n} {cin}->{cout}]", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(5)
+    V = n[0] * n[1] * n[2]
+    x = torch.relu(torch.randn(V, cin, generator=gen, device=DEV)).to(torch.bfloat16)
+    g = torch.randn(V, cout, generator=gen, device=DEV).to(torch.bfloat16)
+    G = L.ngapnet_wgrad_parts(*n, cin, cout)
+    part = torch.empty(G * 27 * cin * cout, device=DEV)
+    dw = torch.empty(27, cout, cin, device=DEV)
+    unet._enter()
+    rc = L.ngapnet_conv3_wgrad(_p(x), _p(g), _p(dw), _p(part), *n, cin, cout, None)
+    unet._leave()
+    assert rc == 0
+    x64, gt = x.double(), g.double().T.contiguous()
+    num = den = 0.0
+    for t in range(27):
+        ref = gt @ _shifted(x64, n, t)
+        num += float((dw[t].double() - ref).square().sum())
+        den += float(ref.square().sum())
+    err = (num / den) ** 0.5
+    lim = 2.0 ** -24 * (V / 32 / G / 3.5 + G / 8) ** 0.5
+    print(f"error {err:.2e}, bound {lim:.2e}", flush=True)
+    assert err <= lim
