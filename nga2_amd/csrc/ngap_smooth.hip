@@ -1483,9 +1483,11 @@ __global__ void __launch_bounds__(256) k_dense_t(int n, const double *__restrict
 // of them through the dense coarsest solve back to its post-smoothing, in one
 // workgroup of 1024 threads with a barrier between phases. On these levels
 // every launch of the per-level kernels costs a few microseconds of latency for
-// a few thousand cells of work. Every sum keeps the order of the per-level
-// kernels, and sweeps in place equal the out-of-place ones (each colour reads
-// only the other colour), so the results are theirs bit for bit.
+// a few thousand cells of work. Every sum keeps the order and the roundings of
+// the per-level kernels of short rows, and sweeps in place equal the out-of-place
+// ones (each colour reads only the other colour), so the results are theirs bit
+// for bit (rows of 64 FP64 or 128 FP32 cells and more: but for the rounding of
+// the residual's first two products, see bottom_fits).
 //
 // A phase is bound by latency: its loads, the chain of six multiply-adds, the
 // division, the barrier. So everything is in LDS: at the start the coefficients
@@ -1804,9 +1806,18 @@ __global__ void __launch_bounds__(BT_THREADS) k_bottom(BotArgs<T> a) {
 
 }  // namespace
 
+// levels whose rows are long enough for the row-wave kernels (k_stencil_rw)
+template <typename T>
+static bool row_waves(const Geo &g) {
+    constexpr int CPL = 16 / sizeof(T);
+    return g.n0 % CPL == 0 && g.n0 >= 32 * CPL;
+}
+
 // Whether levels of these shapes, first to coarsest, are the bottom kernel's:
 // one cell of a colour per thread, and all arrays in its LDS (2048 FP32 or 1024
-// FP64 cells in the first level of a halving sequence).
+// FP64 cells in the first level of a halving sequence). Beyond 1024 cells, levels
+// with rows long enough for k_stencil_rw stay out: that kernel's residual fuses the
+// first two products the other way round, so the cycle's bits would change.
 static long long bottom_places(const Geo &g) { return 2LL * ((g.n0 + 1) / 2) * g.n1 * g.n2; }
 
 template <typename T>
@@ -1814,7 +1825,7 @@ bool bottom_fits(const Geo *g, int n) {
     long long cap = 0, cells = 0;
     for (int l = 0; l < n; l++) {
         const long long q = bottom_places(g[l]);
-        if (l < n - 1 && q > 2 * BT_THREADS) return false;
+        if (l < n - 1 && (q > 2 * BT_THREADS || (g[l].N > 1024 && row_waves<T>(g[l])))) return false;
         cap = std::max(cap, q);
         cells += g[l].N;
     }
@@ -1898,7 +1909,7 @@ template <typename T>
 ApplyCfg apply_cfg(const Geo &g) {
     constexpr int CPL = 16 / sizeof(T);
     ApplyCfg a{};
-    if (g.n0 % CPL == 0 && g.n0 >= 32 * CPL) {
+    if (row_waves<T>(g)) {
         a.rw = true;
         a.gx = (g.n0 + 64 * CPL - 1) / (64 * CPL);
         a.gy = (g.n1 + 3) / 4;
