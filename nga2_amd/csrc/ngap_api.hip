@@ -51,10 +51,6 @@ __device__ __forceinline__ void decomp0(const Geo &g, long long p, int &i, int &
     j = (int)(r - (unsigned)k * (unsigned)g.n1);
 }
 
-__device__ __forceinline__ long long lin0(const Geo &g, int i, int j, int k) {
-    return (long long)i + (long long)g.n0 * ((long long)j + (long long)g.n1 * k);
-}
-
 // ---------------------------------------------------------------- setup kernels
 
 // Level-0 symmetric storage from the ghosted AoS opr (hypre_str_class.f90:

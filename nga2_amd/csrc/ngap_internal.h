@@ -24,7 +24,7 @@ void launch_apply_x32(hipStream_t s, const Geo &g, const double *c, const double
 // <= 128 cells run whole-row tiles (k_sweep_row) unless tiles is set.
 template <typename T>
 void launch_sweep(hipStream_t s, const Geo &g, const T *c, const T *a0, const T *a1, const T *a2, const T *f,
-                  const T *vin, T *vout, int c1, bool one_cell = false);
+                  const T *vin, T *vout, int c1, bool tiles = false);
 // three transfers in one launch between level g[0] and g[3] (directions dirs[0..2],
 // weights pm, pp of levels 1..3); false, with nothing launched, unless the
 // directions all differ
