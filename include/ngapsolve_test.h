@@ -33,6 +33,9 @@ int ngapt_nlevels(const ngap_t *h);
  * NGAP_ERR_ALLOC (n = 0: none), so a test can check that a setup which ran
  * out of memory part-way leaves the handle usable by the next setup. */
 int ngapt_fail_alloc(ngap_t *h, int n);
+/* How the cycle runs the sweeps of a level of n3 cells (per3: periodic): 0 one by
+ * one, 1 in pairs with one cell per lane, 2 in pairs with two. Host only. */
+int ngapt_pairs(const int *n3, const int *per3, int prec);
 int ngapt_level_info(const ngap_t *h, int l, int *dims3, int *cdir);
 int ngapt_level_coefs(const ngap_t *h, int l, double *c, double *ax, double *ay, double *az, double *pm, double *pp);
 int ngapt_apply(ngap_t *h, int l, int prec, const double *x, double *y);
@@ -42,7 +45,7 @@ int ngapt_apply(ngap_t *h, int l, int prec, const double *x, double *y);
  * bits 1 and 2: the first two sweeps from a zero iterate in one launch;
  * without bits 1 and 2, bit 3: the 64-wide tiled sweep kernel also on levels
  * whose rows fit one workgroup row, and bit 4: the sweep kernel itself from a
- * zero iterate */
+ * zero iterate; with bit 2, bit 3: the pair with one cell per lane on every level */
 int ngapt_rbgs(ngap_t *h, int l, int prec, const double *f, double *v, int order);
 /* residual + restriction, prolongation + correction of level l; prec bit 0:
  * FP32, bit 1: the one-cell-per-thread transfer kernels on every level (the

@@ -1148,17 +1148,6 @@ void launch_bottom_levels(ngap_t *h, int lb) {
     launch_bottom<T>(h->stream, a);
 }
 
-// Levels whose sweeps run in fused pairs. With k_sweep2_pair (pair_form) from
-// 2^19 cells on: 256^3 channel, FP32 V(2,2), 22.17 ms a solve with pairs on the
-// fine level only, 21.05 from 2^23, 20.21 from 2^20, 20.10 from 2^19 and 2^18,
-// 20.25 from 2^16 (implicit 128^3: 5.17, 5.24, 4.90, 4.78, 4.84, 4.88 ms); below,
-// a launch has too few planes per chunk and too few workgroups. With k_sweep2 on
-// the largest levels only: at 256^3 the pair took 244 us against 2 x 131, and it
-// was slower on the smaller ones.
-template <typename T>
-static bool pairs_on(const Geo &g) {
-    return g.N >= (pair_form<T>(g) ? 1LL << 19 : 1LL << 24);
-}
 // Levels whose first pre-smoothing sweep (from a zero iterate) runs as the
 // whole-row sweep kernel rather than the stencil form: rows of <= 128 cells,
 // >= 2^20 cells. The stencil reads f and c at every neighbour to form f / c;
@@ -2687,6 +2676,16 @@ int ngap_last_stats(const ngap_t *h, ngap_stats *s) {
 // ------------------------------------------------------------ test hooks
 
 int ngapt_nlevels(const ngap_t *h) { return (h && h->setup_done) ? h->nlev : -1; }
+
+int ngapt_pairs(const int *n3, const int *per3, int prec) {
+    if (!n3 || !per3) return -1;
+    Geo g{};
+    g.n0 = n3[0], g.n1 = n3[1], g.n2 = n3[2];
+    g.p0 = per3[0], g.p1 = per3[1], g.p2 = per3[2];
+    g.N = (long long)g.n0 * g.n1 * g.n2;
+    if (!(prec ? pairs_on<float>(g) : pairs_on<double>(g))) return 0;
+    return (prec ? pair_form<float>(g) : pair_form<double>(g)) ? 2 : 1;
+}
 
 int ngapt_fail_alloc(ngap_t *h, int n) {
     if (!h || n < 0) return NGAP_ERR_ARG;

@@ -34,13 +34,32 @@ bool launch_gather3(hipStream_t s, const Geo *g, const int *dirs, const T *const
 template <typename T>
 bool launch_prolong3(hipStream_t s, const Geo *g, const int *dirs, const T *const *pm, const T *const *pp,
                      const T *vc, const T *vin, T *vout);
-// true where launch_sweep2 can take k_sweep2_pair: FP32, even row length, and
-// even counts where periodic (an odd one has no red-black order across the wrap;
-// k_sweep2 colours by the wrapped index). Offsets in a plane are 32 bits of bytes.
+// true where launch_sweep2 takes k_sweep2_pair: FP32, even row length (x pairs),
+// and no periodic direction of one cell in y or z (other periodic counts are even
+// on every level; k_sweep2_pair colours by the unwrapped index). Offsets in a
+// plane are 32 bits of bytes. And enough planes: a workgroup does at least 12
+// steps for up to 6 planes, so on few planes the kernel is the better one only
+// while its tiles run in few rounds on 256 CUs. Post- and pre-smoothing pair
+// together against four single sweeps, us: 1024^2 x 1 110 and 70, x 2 110 and 89,
+// x 3 112 and 107, x 4 114 and 124 (817 tiles); 720 x 728 x 2 58 and 59, x 3 58
+// and 71 (403 tiles); 600 x 500 x 2 31 and 42 (231 tiles).
+constexpr int PAIR_CX = 56, PAIR_CY = 24;  // output cells of its tiles
 template <typename T>
 inline bool pair_form(const Geo &g) {
+    const long long tiles = (long long)((g.n0 + PAIR_CX - 1) / PAIR_CX) * ((g.n1 + PAIR_CY - 1) / PAIR_CY);
     return sizeof(T) == 4 && g.n0 % 2 == 0 && !(g.p1 && (g.n1 & 1)) && !(g.p2 && (g.n2 & 1)) &&
-           (long long)g.n0 * g.n1 < (1LL << 30);
+           (long long)g.n0 * g.n1 < (1LL << 30) && (g.n2 >= 4 || tiles <= 256LL * (g.n2 - 1));
+}
+// Levels whose sweeps run in fused pairs. With k_sweep2_pair from 2^19 cells on:
+// 256^3 channel, FP32 V(2,2), 22.17 ms a solve with pairs on the fine level only,
+// 21.05 from 2^23, 20.21 from 2^20, 20.10 from 2^19 and 2^18, 20.25 from 2^16
+// (implicit 128^3: 5.17, 5.24, 4.90, 4.78, 4.84, 4.88 ms); below, a launch has too
+// few planes per chunk and too few workgroups. With k_sweep2 on the largest levels
+// only: at 256^3 the pair took 244 us against 2 x 131, and it was slower on the
+// smaller ones.
+template <typename T>
+inline bool pairs_on(const Geo &g) {
+    return g.N >= (pair_form<T>(g) ? 1LL << 19 : 1LL << 24);
 }
 // two fused sweeps of the same colour order (vin != vout); one_cell: the
 // one-cell-per-lane kernel on every level

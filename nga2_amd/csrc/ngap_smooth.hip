@@ -1134,6 +1134,7 @@ __global__ void __launch_bounds__(256) k_prolong3(Chain<T> ch, const T *__restri
 // roundings of k_sweep2, so bit-identical to it. In a 256^3 solve 247 -> 145 us,
 // from zero 209 -> 142 us.
 constexpr int PX = 64, PY = 32, PR = 4;
+static_assert(PX - 2 * PR == PAIR_CX && PY - 2 * PR == PAIR_CY, "pair_form counts these tiles");
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 

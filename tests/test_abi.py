@@ -61,6 +61,29 @@ def test_tiled_convolutions_refuse_empty_and_ragged_boxes(call, dims):
     assert p.stdout.split()[-1] == "-1", p.stdout
 
 
+@pytest.mark.parametrize("n,per,want", [
+    ((256, 256, 256), (1, 0, 1), 2),
+    ((1024, 1024, 1), (0, 0, 0), 0),    # 817 tiles of 12 steps for one plane: two single sweeps take 0.6 of it
+    ((2048, 2048, 1), (0, 0, 0), 0),
+    ((1024, 1024, 2), (1, 1, 1), 0),
+    ((1024, 1024, 3), (0, 0, 0), 0),
+    ((1024, 1024, 4), (0, 0, 0), 2),
+    ((512, 512, 2), (0, 0, 0), 2),      # one round of tiles
+    ((720, 728, 3), (0, 0, 0), 2),      # two rounds
+    ((4096, 4096, 1), (0, 0, 0), 1),    # 2^24 cells: the pair with one cell per lane
+    ((1024, 1024, 1), (1, 1, 1), 0),
+    ((1024, 1, 1024), (1, 1, 1), 0),    # one periodic cell
+    ((129, 129, 129), (0, 0, 0), 0),    # odd rows
+    ((64, 64, 64), (1, 1, 1), 0),       # fewer than 2^19 cells
+])
+def test_levels_whose_sweeps_run_in_pairs(n, per, want):
+    """Thin levels take the pair only where it was measured to be the faster form."""
+    a, b = (ctypes.c_int * 3)(*n), (ctypes.c_int * 3)(*per)
+    L = _lib.lib()
+    assert L.ngapt_pairs(a, b, 1) == want
+    assert L.ngapt_pairs(a, b, 0) == (1 if n[0] * n[1] * n[2] >= 2 ** 24 else 0)
+
+
 def test_strerror_and_defaults_without_gpu():
     assert _lib.strerror(0) == "ok"
     assert "setup" in _lib.strerror(_lib.ERR_NOT_SETUP)

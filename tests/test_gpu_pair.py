@@ -2,7 +2,8 @@
 form on every level of boxes at the edges of its tiles (output core 56 x 24
 cells, chunks of whole 6 planes): cores filled exactly, one pair or row more,
 boxes smaller than the ring, directions of two cells, periodic and walled. Both
-issue the same operations in the same order: the same bits.
+issue the same operations in the same order: the same bits. (Levels with odd
+rows, one plane or one periodic cell in y or z have the one-cell form only.)
 """
 import numpy as np
 import pytest
@@ -18,11 +19,12 @@ SHAPES = [
     ((112, 49, 13), (True, False, False)),
     ((64, 32, 12), (True, True, True)),
     ((2, 2, 2), (True, True, True)),
-    ((2, 3, 1), (False, False, False)),
+    ((2, 3, 2), (False, False, False)),
     ((6, 4, 34), (False, True, True)),
     ((62, 8, 5), (False, True, False)),
     ((200, 70, 40), (False, False, True)),
-    ((30, 6, 8), (False, True, True)),       # 3 periodic rows on a coarse level: the one-cell form
+    ((30, 6, 8), (False, True, True)),       # 6 periodic rows: a tile wraps around the box five times
+    ((48, 64, 24), (True, True, False)),     # periodic directions that coarsen
 ]
 
 
