@@ -200,7 +200,7 @@ __global__ void __launch_bounds__(PT) k_sync_dir(Grid g, int ax, double *a) {
 // digit-reversed order and stay there: the operator's transform has the same
 // order, the divide is pointwise, and the inverse runs the passes backwards.
 constexpr int FFT_MAX = 1024;  // 8 lines of 16 bytes a cell: 128 KB of LDS
-constexpr int FT = 256;                // threads of a workgroup at most
+constexpr int FT = 256;                // threads of a row workgroup at most
 constexpr int LB = 3, LINES = 1 << LB;  // lines of a column tile
 struct FftDim {
     int n, np;
@@ -345,8 +345,15 @@ __device__ __forceinline__ void by_radix(int r, Run run) {
 // pass, the library's 82; the divide (405 MB) 103 us, two library passes and a
 // divide 221.
 enum { FWD, INV, DIVIDE };
+// Threads: one per radix-8 butterfly of a pass, at most 256, or so many that the
+// workgroups that fit a CU's LDS fill its 16 waves (8 of a BIG kernel's): lines of
+// more than 568 cells leave one and with 256 threads its latency bare
+// (1024^2 x 32: 1080 us a solve with 256 threads, 917 now; 16 x 1024 x 16: 105 and
+// 79 us, the library 84 to 99). Other counts than powers of two leave SIMDs uneven
+// (300^3 with 320 threads: 788 us against 685).
+constexpr size_t CU_LDS = 160 * 1024;
 template <int MODE, bool BIG>
-__global__ void __launch_bounds__(FT, BIG ? 2 : 4) k_fft_col(FftDim D, const double2 *__restrict__ finv, double2 *a, int nlines,
+__global__ void __launch_bounds__(BIG ? 512 : 1024) k_fft_col(FftDim D, const double2 *__restrict__ finv, double2 *a, int nlines,
                                                 long long es, long long ostride, int pitch, int nxh,
                                                 double scale) {
     extern __shared__ double2 sm[];
@@ -678,7 +685,7 @@ int row_pairs(const Grid &g) {
     while (pr > 1 && (long long)g.ny * g.nz / (2 * pr) < 512) pr /= 2;
     return pr;
 }
-int threads_for(int cells) { return std::min(FT, std::max(64, (cells / 8 + 63) / 64 * 64)); }
+int threads_for(int cells, int most = FT) { return std::min(most, std::max(64, (cells / 8 + 63) / 64 * 64)); }
 size_t row_lds(int n, int pr) { return sizeof(double2) * (n + (size_t)pr * (n + n / 8 + 1)) + sizeof(short) * n; }
 size_t col_lds(int n) { return sizeof(double2) * (n + (size_t)n * LINES); }
 
@@ -686,6 +693,12 @@ bool big(const FftDim &D) {
     for (int p = 0; p < D.np; p++)
         if (D.r[p] == 7 || D.r[p] > 8) return true;
     return false;
+}
+
+int col_threads(const FftDim &D) {
+    const size_t fit = CU_LDS / col_lds(D.n);
+    const int most = big(D) ? (fit > 1 ? 256 : 512) : (fit > 2 ? 256 : (fit > 1 ? 512 : 1024));
+    return threads_for(D.n * LINES, most);
 }
 
 void rows_fwd(ngap_fft *F, const double *src, double2 *dst) {
@@ -713,7 +726,7 @@ void cols(ngap_fft *F, int ax, double2 *a, double scale) {
     const long long row = F->pitch, plane = row * g.ny;
     const int lines = (int)(ax == 1 ? row : plane);
     hipLaunchKernelGGL(col_kernel<MODE>(F->D[ax]), dim3((unsigned)((lines + LINES - 1) / LINES), ax == 1 ? g.nz : 1),
-                       dim3(threads_for(n * LINES)), col_lds(n), F->s, F->D[ax], (const double2 *)F->d_finv, a, lines,
+                       dim3(col_threads(F->D[ax])), col_lds(n), F->s, F->D[ax], (const double2 *)F->d_finv, a, lines,
                        ax == 1 ? row : plane, plane, F->pitch, F->nxh, scale);
 }
 

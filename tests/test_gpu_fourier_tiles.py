@@ -27,7 +27,12 @@ SHAPES = [
     ((169, 7, 3), 1),        # an odd number of rows
     ((126, 1, 9), 1),        # no y transform
     ((8, 1024, 2), 1),       # 144 KB of LDS a workgroup
+    ((4, 2, 512), 1),        # 72 KB: 512 threads
+    ((4, 1001, 3), 1),       # 7 x 11 x 13 in 141 KB: 512 threads of more registers
     ((1024, 2, 1), 1),
+    ((143, 63, 49), 1),      # three row pairs a workgroup, the last with one and a half
+    ((1001, 65, 32), 1),     # long rows, two pairs a workgroup
+    ((1024, 33, 64), 1),
     ((16, 16, 17), 1),       # a prime factor above 13: the library
     ((8, 1026, 2), 1),
     ((1, 16, 24), 1),        # no x transform: the library
