@@ -730,14 +730,17 @@ void cols(ngap_fft *F, int ax, double2 *a, double scale) {
                        ax == 1 ? row : plane, plane, F->pitch, F->nxh, scale);
 }
 
-// more than 64 KB of LDS is asked for by name
+// More than 64 KB of LDS is asked for by name. The limit belongs to the kernel, not
+// to a handle: always the largest tile's, so that no handle lowers another's.
 bool allow_lds(const FftDim &D) {
-    const int lds = (int)col_lds(D.n);
-    if (lds <= 65536) return true;
+    if (col_lds(D.n) <= 65536) return true;
     const void *k[] = {(const void *)col_kernel<FWD>(D), (const void *)col_kernel<INV>(D),
                        (const void *)col_kernel<DIVIDE>(D)};
     for (const void *q : k)
-        if (hipFuncSetAttribute(q, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return false;
+        if (hipFuncSetAttribute(q, hipFuncAttributeMaxDynamicSharedMemorySize, (int)col_lds(FFT_MAX)) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
     return true;
 }
 
@@ -871,7 +874,8 @@ int ngap_fft_create(ngap_fft **fp, const ngap_grid *gr, int nst, const int *stc)
     for (int d = 0; d + 1 < r; d++) F->M *= dims[d];
     if (r > 0) F->M *= dims[r - 1] / 2 + 1;
     F->own = g.nx > 1 && factor(g.nx, &F->D[0]) && (g.ny == 1 || factor(g.ny, &F->D[1])) &&
-             (g.nz == 1 || factor(g.nz, &F->D[2])) && (long long)g.ny * g.nz < (1LL << 30) && g.nz < 65536;
+             (g.nz == 1 || factor(g.nz, &F->D[2])) && (long long)g.ny * g.nz < (1LL << 30) && g.nz < 65536 &&
+             (g.ny == 1 || allow_lds(F->D[1])) && (g.nz == 1 || allow_lds(F->D[2]));  // else the library
     if (F->own) {
         F->nxh = g.nx / 2 + 1;
         F->pitch = (F->nxh + 7) / 8 * 8;
@@ -898,10 +902,8 @@ int ngap_fft_create(ngap_fft **fp, const ngap_grid *gr, int nst, const int *stc)
     if (!rc) rc = dalloc(F, &F->d_spec, (size_t)F->M);
     if (!rc) rc = dalloc(F, &F->d_finv, (size_t)F->M);
     if (!rc && hipMemcpy(F->d_stc, stc, sizeof(int) * 3 * nst, hipMemcpyHostToDevice) != hipSuccess) rc = NGAP_ERR_HIP;
-    for (int d = 0; d < 3 && !rc && F->own; d++) {
+    for (int d = 0; d < 3 && !rc && F->own; d++)
         if (F->D[d].n) rc = plan_dim(F, &F->D[d]);
-        if (!rc && d > 0 && F->D[d].n && !allow_lds(F->D[d])) rc = NGAP_ERR_HIP;
-    }
     if (!rc && r > 0 && !F->own) {
         if (hipfftPlanMany(&F->fwd, r, dims, rembed, rstride, (int)g.No, cembed, 1, (int)F->M, HIPFFT_D2Z, 1) !=
             HIPFFT_SUCCESS)

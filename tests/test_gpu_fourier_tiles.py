@@ -40,17 +40,25 @@ SHAPES = [
 ]
 
 
-@pytest.mark.parametrize("n,no", SHAPES)
-def test_solve_matches_oracle(n, no):
-    print(f"\n[fourier tiles {n} ghosts {no}]", flush=True)
+def problem(n, no):
     per = tuple(m > 1 for m in n)
     cfg = Config(*(uniform(m, m / max(n)) for m in n), no=no, xper=per[0], yper=per[1], zper=per[2])
     opr = incomp.laplacian(incomp.Metrics(cfg))
     rng = np.random.default_rng(11)
     rhs, sol0 = (np.asfortranarray(rng.standard_normal(cfg.shape)) for _ in range(2))
     ref = F3.solve(cfg, F3.setup(cfg, opr, STC7, fourier.circ_tol(cfg)), rhs, sol0)
+    return cfg, opr, rhs, sol0, ref
+
+
+def up(a):
+    return torch.from_numpy(np.ascontiguousarray(a.ravel(order="F"))).cuda()
+
+
+@pytest.mark.parametrize("n,no", SHAPES)
+def test_solve_matches_oracle(n, no):
+    print(f"\n[fourier tiles {n} ghosts {no}]", flush=True)
+    cfg, opr, rhs, sol0, ref = problem(n, no)
     ds = fourier.DeviceFourier(cfg)
-    up = lambda a: torch.from_numpy(np.ascontiguousarray(a.ravel(order="F"))).cuda()
     ds.setup(up(opr))
     d_rhs, d_sol = up(rhs), up(sol0)
     ds.solve(d_rhs, d_sol)
@@ -63,3 +71,22 @@ def test_solve_matches_oracle(n, no):
     assert np.array_equal(chk, got)
     assert torch.equal(d_rhs, up(rhs))
     ds.destroy()
+
+
+def test_handles_of_long_and_shorter_lines():
+    """The LDS a kernel may use is a limit of the kernel: a handle made later
+    for shorter lines (still over 64 KB) leaves an older one's as it is."""
+    made = []
+    for n in ((8, 1024, 2), (8, 576, 2)):
+        print(f"\n[fourier handles {n}]", flush=True)
+        cfg, opr, rhs, sol0, ref = problem(n, 1)
+        ds = fourier.DeviceFourier(cfg)
+        ds.setup(up(opr))
+        made.append((ds, n, cfg, rhs, sol0, ref))
+    for ds, n, cfg, rhs, sol0, ref in made:
+        d_rhs, d_sol = up(rhs), up(sol0)
+        ds.solve(d_rhs, d_sol)
+        got = d_sol.cpu().numpy().reshape(cfg.shape, order="F")
+        tol = max(1e-12, 8 * 2.0 ** -52 * (max(n) / np.pi) ** 2)
+        assert np.abs(got - ref).max() <= tol * np.abs(ref).max()
+        ds.destroy()
