@@ -1156,15 +1156,15 @@ void launch_bottom_levels(ngap_t *h, int lb) {
 constexpr long long ZSWEEP_MIN_CELLS = 1LL << 20;
 
 // The three transfers below level l as one launch: l + 1 and l + 2 are skipped
-// levels, l + 3 is at most `top`.
+// levels, l + 3 is at most `top`, and the three directions differ (order 0: not so).
 template <typename T>
 struct Skip3 {
     Geo g[4];
-    int dirs[3];
     const T *pm[3], *pp[3];
-    bool on = false;
+    int order = 0;
     Skip3(ngap_t *h, int l, int top) {
         if (l + 3 > top || h->lev[l + 1].relax || h->lev[l + 2].relax) return;
+        int dirs[3];
         g[0] = h->lev[l].g;
         for (int i = 0; i < 3; i++) {
             dirs[i] = h->lev[l + i].cdir;
@@ -1173,7 +1173,7 @@ struct Skip3 {
             pm[i] = D.pm;
             pp[i] = D.pp;
         }
-        on = dirs[0] != dirs[1] && dirs[0] != dirs[2] && dirs[1] != dirs[2];
+        order = chain_order(dirs);
     }
 };
 
@@ -1203,7 +1203,8 @@ void vcycle(ngap_t *h, const T *f0, T *v0) {
     std::vector<char> bridged(nl, 0);  // skipped levels that a Skip3 launch passes over
     auto restrict_from = [&](int l, const T *r) {
         const Skip3<T> k(h, l, top);
-        if (k.on && launch_gather3<T>(s, k.g, k.dirs, k.pm, k.pp, r, data<T>(h->lev[l + 3]).f)) {
+        if (k.order) {
+            launch_gather3<T>(s, k.g, k.order, k.pm, k.pp, r, data<T>(h->lev[l + 3]).f);
             bridged[l + 1] = bridged[l + 2] = 1;
             return;
         }
@@ -1213,7 +1214,7 @@ void vcycle(ngap_t *h, const T *f0, T *v0) {
     auto prolong_to = [&](int l, const T *vin, T *vout) {
         if (l + 1 < nl && bridged[l + 1]) {
             const Skip3<T> k(h, l, top);
-            launch_prolong3<T>(s, k.g, k.dirs, k.pm, k.pp, data<T>(h->lev[l + 3]).v, vin, vout);
+            launch_prolong3<T>(s, k.g, k.order, k.pm, k.pp, data<T>(h->lev[l + 3]).v, vin, vout);
             return;
         }
         LevelData<T> &DC = data<T>(h->lev[l + 1]);

@@ -25,15 +25,16 @@ void launch_apply_x32(hipStream_t s, const Geo &g, const double *c, const double
 template <typename T>
 void launch_sweep(hipStream_t s, const Geo &g, const T *c, const T *a0, const T *a1, const T *a2, const T *f,
                   const T *vin, T *vout, int c1, bool tiles = false);
-// three transfers in one launch between level g[0] and g[3] (directions dirs[0..2],
-// weights pm, pp of levels 1..3); false, with nothing launched, unless the
-// directions all differ
+// three transfers in one launch between level g[0] and g[3] (weights pm, pp of
+// levels 1..3) along the directions dirs[0..2], whose chain_order is not 0
+inline int chain_order(const int *dirs) {  // 0 unless the three differ
+    return dirs[0] != dirs[1] && dirs[0] != dirs[2] && dirs[1] != dirs[2] ? 3 * dirs[0] + dirs[1] : 0;
+}
 template <typename T>
-bool launch_gather3(hipStream_t s, const Geo *g, const int *dirs, const T *const *pm, const T *const *pp, const T *r,
-                    T *fc);
+void launch_gather3(hipStream_t s, const Geo *g, int order, const T *const *pm, const T *const *pp, const T *r, T *fc);
 template <typename T>
-bool launch_prolong3(hipStream_t s, const Geo *g, const int *dirs, const T *const *pm, const T *const *pp,
-                     const T *vc, const T *vin, T *vout);
+void launch_prolong3(hipStream_t s, const Geo *g, int order, const T *const *pm, const T *const *pp, const T *vc,
+                     const T *vin, T *vout);
 // true where launch_sweep2 takes k_sweep2_pair: FP32, even row length (x pairs),
 // and no periodic direction of one cell in y or z (other periodic counts are even
 // on every level; k_sweep2_pair colours by the unwrapped index). Offsets in a

@@ -2187,11 +2187,9 @@ void launch_prolong_to(hipStream_t s, const Geo &F, const Geo &C, int d, const T
         hipLaunchKernelGGL((k_prolong_t<T, 2>), grid, dim3(tx, ty), 0, s, F, C, pm, pp, vc, vin, vout);
 }
 
-// directions of a chain: -1 unless all three differ
-static int chain_order(const int *d) { return d[0] != d[1] && d[0] != d[2] && d[1] != d[2] ? 3 * d[0] + d[1] : -1; }
-
+// order: chain_order of the directions
 template <typename T, typename F>
-static bool launch_chain(const Geo *g, const int *dirs, const T *const *pm, const T *const *pp, F launch) {
+static void launch_chain(const Geo *g, int order, const T *const *pm, const T *const *pp, F launch) {
     Chain<T> ch;
     for (int i = 0; i < 4; i++) ch.g[i] = g[i];
     for (int i = 0; i < 3; i++) ch.pm[i] = pm[i], ch.pp[i] = pp[i];
@@ -2199,30 +2197,30 @@ static bool launch_chain(const Geo *g, const int *dirs, const T *const *pm, cons
     const int tx = std::min(64, pow2ceil(g[3].n0)), ty = 64 / tx;
     const dim3 grid((g[3].n0 + tx - 1) / tx, (g[3].n1 + ty - 1) / ty, g[3].n2), block(tx, ty);
     using std::integral_constant;
-    switch (chain_order(dirs)) {
-        case 1: launch(ch, grid, block, integral_constant<int, 0>(), integral_constant<int, 1>(), integral_constant<int, 2>()); break;
-        case 2: launch(ch, grid, block, integral_constant<int, 0>(), integral_constant<int, 2>(), integral_constant<int, 1>()); break;
-        case 3: launch(ch, grid, block, integral_constant<int, 1>(), integral_constant<int, 0>(), integral_constant<int, 2>()); break;
-        case 5: launch(ch, grid, block, integral_constant<int, 1>(), integral_constant<int, 2>(), integral_constant<int, 0>()); break;
-        case 6: launch(ch, grid, block, integral_constant<int, 2>(), integral_constant<int, 0>(), integral_constant<int, 1>()); break;
-        case 7: launch(ch, grid, block, integral_constant<int, 2>(), integral_constant<int, 1>(), integral_constant<int, 0>()); break;
-        default: return false;
+    using X = integral_constant<int, 0>;
+    using Y = integral_constant<int, 1>;
+    using Z = integral_constant<int, 2>;
+    switch (order) {
+        case 1: launch(ch, grid, block, X(), Y(), Z()); break;
+        case 2: launch(ch, grid, block, X(), Z(), Y()); break;
+        case 3: launch(ch, grid, block, Y(), X(), Z()); break;
+        case 5: launch(ch, grid, block, Y(), Z(), X()); break;
+        case 6: launch(ch, grid, block, Z(), X(), Y()); break;
+        default: launch(ch, grid, block, Z(), Y(), X()); break;
     }
-    return true;
 }
 
 template <typename T>
-bool launch_gather3(hipStream_t s, const Geo *g, const int *dirs, const T *const *pm, const T *const *pp, const T *r,
-                    T *fc) {
-    return launch_chain<T>(g, dirs, pm, pp, [&](const Chain<T> &ch, dim3 grid, dim3 block, auto a, auto b, auto c) {
+void launch_gather3(hipStream_t s, const Geo *g, int order, const T *const *pm, const T *const *pp, const T *r, T *fc) {
+    launch_chain<T>(g, order, pm, pp, [&](const Chain<T> &ch, dim3 grid, dim3 block, auto a, auto b, auto c) {
         hipLaunchKernelGGL((k_gather3<T, a(), b(), c()>), grid, block, 0, s, ch, r, fc);
     });
 }
 
 template <typename T>
-bool launch_prolong3(hipStream_t s, const Geo *g, const int *dirs, const T *const *pm, const T *const *pp,
-                     const T *vc, const T *vin, T *vout) {
-    return launch_chain<T>(g, dirs, pm, pp, [&](const Chain<T> &ch, dim3 grid, dim3 block, auto a, auto b, auto c) {
+void launch_prolong3(hipStream_t s, const Geo *g, int order, const T *const *pm, const T *const *pp, const T *vc,
+                     const T *vin, T *vout) {
+    launch_chain<T>(g, order, pm, pp, [&](const Chain<T> &ch, dim3 grid, dim3 block, auto a, auto b, auto c) {
         hipLaunchKernelGGL((k_prolong3<T, a(), b(), c()>), grid, block, 0, s, ch, vc, vin, vout);
     });
 }
@@ -2252,10 +2250,10 @@ template void launch_bottom<float>(hipStream_t, const BotArgs<float> &);
                                    T *, bool);                                                                     \
     template void launch_prolong_to<T>(hipStream_t, const Geo &, const Geo &, int, const T *, const T *,           \
                                        const T *, const T *, T *, bool);                                           \
-    template bool launch_gather3<T>(hipStream_t, const Geo *, const int *, const T *const *, const T *const *,     \
-                                    const T *, T *);                                                               \
-    template bool launch_prolong3<T>(hipStream_t, const Geo *, const int *, const T *const *, const T *const *,    \
-                                     const T *, const T *, T *);                                                   \
+    template void launch_gather3<T>(hipStream_t, const Geo *, int, const T *const *, const T *const *, const T *,  \
+                                    T *);                                                                          \
+    template void launch_prolong3<T>(hipStream_t, const Geo *, int, const T *const *, const T *const *, const T *, \
+                                     const T *, T *);                                                              \
     template void launch_dense<T, T>(hipStream_t, int, const double *, const T *, T *);
 INST(double)
 INST(float)
