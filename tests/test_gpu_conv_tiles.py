@@ -140,3 +140,31 @@ def test_weight_gradient_sums_stay_short(n, cin, cout):
     lim = 2.0 ** -24 * (V / 32 / G / 3.5 + G / 8) ** 0.5
     print(f"error {err:.2e}, bound {lim:.2e}", flush=True)
     assert err <= lim
+
+
+def test_planes_beyond_4_gib():
+    """Planes of 4 GiB and more take 64-bit offsets. The input repeats a smaller
+    box 12 times in y, so the output repeats that box's, bit for bit; an offset
+    that wrapped at 2^32 bytes would be 8192 rows off, no multiple of the box."""
+    from nga2_amd import unet
+
+    L = unet.lib()
+    nx, ny, nz, c, reps = 8192, 684, 4, 32, 12
+    assert nx * ny * reps * c * 2 >= 2 ** 32 and 2 ** 32 // (nx * c * 2) % ny != 0
+    print("\n[conv planes beyond 4 GiB]", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.randn(nz, 1, ny, nx * c, generator=gen, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(27, c, c, generator=gen, device=DEV) / (27 * c) ** 0.5).to(torch.bfloat16)
+    want = torch.empty_like(x)
+    big = x.expand(nz, reps, ny, nx * c).contiguous()
+    got = torch.empty_like(big)
+    unet._enter()
+    rc = L.ngapnet_conv3_fwd(_p(x), _p(w), None, _p(want), nx, ny, nz, c, c, 1, None)
+    rc |= L.ngapnet_conv3_fwd(_p(big), _p(w), None, _p(got), nx, ny * reps, nz, c, c, 1, None)
+    unet._leave()
+    assert rc == 0
+    assert float(want.float().abs().max()) > 0
+    for r in range(reps):
+        assert torch.equal(got[:, r], want[:, 0]), r
+    del big, got
+    torch.cuda.empty_cache()
