@@ -14,6 +14,8 @@ extern "C" {
 #endif
 int ngapnet_conv3_fwd(const void *in_bf16, const void *wt_bf16, float *out32, void *outb_bf16, int nx, int ny,
                       int nz, int cin, int cout, int relu, void *stream);
+/* Partials (27 * cin * cout floats each) that `part` of ngapnet_conv3_wgrad must have room for; a
+ * launch uses at most so many (fewer where a layer's workgroups need no more). */
 int ngapnet_wgrad_parts(int nx, int ny, int nz, int cin, int cout);
 int ngapnet_conv3_wgrad(const void *in_bf16, const void *dout_bf16, float *dw, float *part, int nx, int ny, int nz,
                         int cin, int cout, void *stream);
